@@ -17,9 +17,10 @@
 // activation row.  The row phases meet through the shared cross-lane and LDS
 // stages and the K slices through the deterministic split-K hand-off.
 //
-// Other shapes: an LDS-tiled fp32 VALU product (64 x 64 tiles, 32-k steps)
-// that dequantizes each weight once per tile with the per-element block
-// index, so any N works.
+// Other shapes: the matrix-core tiles of split.hip (any N and alignment);
+// past their extents, an LDS-tiled fp32 VALU product (64 x 64 tiles, 32-k
+// steps) that dequantizes each weight once per tile with the per-element
+// block index.
 //
 // Activations are f32 or f16 (the reference's two widths); sums are f32 in
 // this library's order, so results agree with the reference to f32 rounding.
@@ -285,6 +286,11 @@ hipError_t launch_int8_any(Device* d, hipStream_t st, const ACT* a, const int8_t
             default: return launch_int8_decode_m<8>(d, st, a, q, s, out, K, N, status);
         }
     }
+    // The matrix-core tiles past the decode shapes: 512 x 4096 x 4096 702 -> 90
+    // us, 16 rows 35, 155 x 1758 x 430 (f32 VALU tiles / here) 98 / 20; the
+    // decode kernel keeps its eight rows (15.6 us there, 34.7 here).
+    if (split_product_supported(M, K, N))
+        return launch_split_int8(d, st, a, sizeof(ACT) == 2, q, s, out, M, K, N);
     dim3 grid((N + QN - 1) / QN, (M + QM - 1) / QM);
     if ((uint64_t)grid.x * 256 >= (1ull << 32) || grid.y > 65535) {
         *status = fail(ACCEL_E_UNSUPPORTED,

@@ -364,6 +364,13 @@ hipError_t launch_int8_product(Device* d, hipStream_t st, const void* a, bool f1
                                const int8_t* quants, const uint16_t* scales, float* out, int M,
                                int K, int N, int* status);
 
+// int8 products on the matrix cores to f32 accuracy (split.hip): any M, N, K
+// and alignment within split_product_supported; needs no workspace.
+bool split_product_supported(int M, int K, int N);
+hipError_t launch_split_int8(const Device* d, hipStream_t st, const void* a, bool f16_act,
+                             const int8_t* quants, const uint16_t* scales, float* out, int M,
+                             int K, int N);
+
 // Device quantizer.
 hipError_t launch_int4_quantize(hipStream_t st, const float* w, int64_t n,
                                 uint32_t* packed, uint16_t* scales, uint16_t* zeros);

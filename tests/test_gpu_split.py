@@ -1,0 +1,90 @@
+"""GPU parity of the matrix-core products of split weights (split.hip): every
+tile, the ragged ends of rows, columns and K, every K-group remainder, and
+infinities, NaNs and tiny values.
+
+Tolerance: rel-L2 1e-5 against the oracle, the path's bound for f32 products.
+The split itself is within 2^-26 of each product; both sides round their sums.
+"""
+import numpy as np
+import pytest
+
+import accel_amd
+import oracle
+from accel_amd import F16, F32
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+F32_TOL = 1e-5
+
+
+def int8_run(dev, a, q, s, M, K, N, f16=False):
+    ab = dev.upload(a.reshape(M, K), F16 if f16 else F32)
+    qb, sb, ob = dev.upload(q.reshape(K, N)), dev.upload(s), dev.alloc((M, N), F32)
+    dev.QuantMatMul(ab, qb, sb, ob)
+    got = ob.numpy()
+    for b in (ab, qb, sb, ob):
+        b.free()
+    return got
+
+
+# (M, K, N): K of no whole stage, fewer stages than K groups, a ragged last
+# stage; one row, one column, column pairs cut by the edge; N odd, even and
+# whole blocks; the tiles 32 x 64, 64 x 64, 64 x 128 and 64 x 256
+INT8 = [(9, 1, 1), (9, 31, 33), (33, 32, 64), (10, 95, 130), (64, 257, 65), (31, 300, 2),
+        (2, 1656, 1359), (130, 511, 96), (257, 1000, 1500), (100, 4100, 4004),
+        (512, 1024, 8192), (2048, 260, 8190), (65, 4097, 16383)]
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("M,K,N", INT8)
+def test_int8_matches_the_oracle(dev, M, K, N, f16):
+    rng = np.random.default_rng(M * 31 + K * 17 + N)
+    a = rng.standard_normal(M * K).astype(np.float32)
+    q, s = oracle.int8_quantize((rng.standard_normal(K * N) * 0.05).astype(np.float32))
+    if f16:
+        a = oracle.to_f16(a)
+    got = int8_run(dev, a, q, s, M, K, N, f16)
+    x = (oracle.f16_to_f32(a) if f16 else a).astype(np.float64).reshape(M, K)
+    w = q.astype(np.float64) * oracle.f16_to_f32(s).astype(np.float64)[np.arange(K * N) // 32]
+    assert rel_l2(got, x @ w.reshape(K, N)) <= F32_TOL
+
+
+def test_int8_infinities_nans_and_the_largest_values_read_as_in_f32(dev):
+    M, K, N = 40, 300, 200
+    rng = np.random.default_rng(3)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    q, s = oracle.int8_quantize((rng.standard_normal(K * N) * 0.05).astype(np.float32))
+    a[3, 7] = np.inf
+    a[5, 9] = -np.inf
+    a[6, 1] = np.nan
+    a[8, 4] = 3.4e38            # rounds to a bf16 infinity; the product is finite
+    q.reshape(K, N)[4, :] = 0
+    q.reshape(K, N)[4, 50] = 1
+    got = int8_run(dev, a, q, s, M, K, N)
+    w = (q.astype(np.float32) * oracle.f16_to_f32(s)[np.arange(K * N) // 32]).reshape(K, N)
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64)
+    for row in (3, 5):
+        k = 7 if row == 3 else 9
+        inf = (w[k] != 0)
+        assert np.array_equal(np.isinf(got[row]), inf)
+        assert np.array_equal(np.sign(got[row][inf]), np.sign(a[row, k] * w[k][inf]))
+        assert np.all(np.isnan(got[row][~inf]))
+    assert np.all(np.isnan(got[6]))
+    assert np.all(np.isfinite(got[8]))
+    rest = np.setdiff1d(np.arange(M), (3, 5, 6))
+    for row in rest:
+        assert rel_l2(got[row], want[row]) <= F32_TOL, row
+
+
+def test_int8_tiny_activations_keep_f32_accuracy(dev):
+    # the last bf16 term of values near 2^-115 is a bf16 subnormal
+    M, K, N = 16, 256, 128
+    rng = np.random.default_rng(4)
+    a = (rng.standard_normal((M, K)) * 2.0 ** -115).astype(np.float32)
+    q, s = oracle.int8_quantize(rng.standard_normal(K * N).astype(np.float32))
+    w = q.astype(np.float64) * oracle.f16_to_f32(s).astype(np.float64)[np.arange(K * N) // 32]
+    got = int8_run(dev, a, q, s, M, K, N)
+    assert rel_l2(got.astype(np.float64) * 2.0 ** 115,
+                  (a.astype(np.float64) * 2.0 ** 115) @ w.reshape(K, N)) <= F32_TOL
