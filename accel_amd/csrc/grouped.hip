@@ -140,10 +140,15 @@ hipError_t launch_segment_offsets(hipStream_t st, const uint32_t* counts, uint32
     return launch_status();
 }
 
-hipError_t launch_grouped_f32(hipStream_t st, const float* x, const float* w,
+hipError_t launch_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,
                               const uint32_t* off, float* out, int E, int T, int K, int N,
                               bool write_padding) {
     if (T == 0 || N == 0) return hipSuccess;
+    // The matrix-core tiles wherever their grid reaches (us, one lane per
+    // element / tiles): 256 rows of 8 experts of 2048 x 4096 1536 / 72, 8 rows
+    // of 4 experts of 156 x 2397 42 / 11.
+    if (split_grouped_supported(E, T, K, N))
+        return launch_split_grouped_f32(d, st, x, w, off, out, E, T, K, N, write_padding);
     dim3 grid((N + 255) / 256, T < 65535 ? T : 65535);
     ACCEL_LAUNCH(tname("grouped_f32_kernel", false), (grouped_f32_kernel<false>), grid,
                  dim3(256), 0, st, x, w, nullptr, nullptr, nullptr, off, out, E, T, K, N,

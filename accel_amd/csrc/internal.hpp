@@ -248,7 +248,7 @@ hipError_t launch_int4_matmul_set(Device* d, hipStream_t st, const float* a, con
 // Grouped products over offsets [E+1] already on the device.
 hipError_t launch_segment_offsets(hipStream_t st, const uint32_t* counts,
                                   uint32_t* offsets, int rows);
-hipError_t launch_grouped_f32(hipStream_t st, const float* x, const float* w,
+hipError_t launch_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,
                               const uint32_t* off, float* out, int E, int T, int K,
                               int N, bool write_padding);
 hipError_t launch_int4_grouped_f32(hipStream_t st, const float* x, Int4Planes w,
@@ -370,6 +370,12 @@ bool split_product_supported(int M, int K, int N);
 hipError_t launch_split_int8(const Device* d, hipStream_t st, const void* a, bool f16_act,
                              const int8_t* quants, const uint16_t* scales, float* out, int M,
                              int K, int N);
+
+// The grouped product over f32 experts the same way, any offsets.
+bool split_grouped_supported(int E, int T, int K, int N);
+hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,
+                                    const uint32_t* off, float* out, int E, int T, int K, int N,
+                                    bool matvec);
 
 // Device quantizer.
 hipError_t launch_int4_quantize(hipStream_t st, const float* w, int64_t n,

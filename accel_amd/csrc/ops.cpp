@@ -805,7 +805,7 @@ int run_grouped_f32(const char* op, int dev, void* stream, const accel_tensor_t*
     uint32_t* off = offsets_in_workspace(d, st, static_cast<const uint32_t*>(counts->data), E,
                                          &status);
     if (!off) return status;
-    hipError_t e = launch_grouped_f32(st, static_cast<const float*>(x->data),
+    hipError_t e = launch_grouped_f32(d, st, static_cast<const float*>(x->data),
                                       static_cast<const float*>(w->data), off,
                                       static_cast<float*>(out->data), (int)E, (int)T, (int)K,
                                       (int)N, matvec);
@@ -2230,7 +2230,7 @@ ACCEL_API int accel_hip_dispatch(int dev, void* stream, const char* kernel,
     if (!d) return ACCEL_E_NO_DEVICE;
     int status = begin_submission(d);
     if (status != ACCEL_OK) return status;
-    hipError_t e = launch_grouped_f32((hipStream_t)stream, static_cast<const float*>(bindings[0]),
+    hipError_t e = launch_grouped_f32(d, (hipStream_t)stream, static_cast<const float*>(bindings[0]),
                                       static_cast<const float*>(bindings[1]),
                                       static_cast<const uint32_t*>(bindings[2]),
                                       static_cast<float*>(const_cast<void*>(bindings[3])),

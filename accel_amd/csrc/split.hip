@@ -1,5 +1,5 @@
 // Products to f32 accuracy on the bf16 matrix cores for weights of the int8
-// format.  Every weight is dequantised exactly as the per-element kernels do
+// format and for the grouped products' plain f32 experts.  Every weight is dequantised exactly as the per-element kernels do
 // it, in f32, and both sides are split into bf16 terms (bf16split.hpp):
 //     f32 rows x weights:  3 x 3 terms, the six products above 2^-27 kept
 //     f16 rows:            2 x 3 terms (an f16 is two terms exactly), five
@@ -67,6 +67,35 @@ struct ActF16 {
 // scales start at a whole block.
 // F and the row's base stay in scalar registers.
 enum { kOdd, kEven, kRows };
+
+// Plain f32 weights (the grouped products' experts, [K, N] each).
+template <int FORM>
+struct F32W {
+    const float* w;
+    __device__ __forceinline__ F32W expert(int e, size_t per) const { return {w + e * per}; }
+    struct Regs { float v[8][2]; };
+    __device__ __forceinline__ void load(Regs& r, int i, uint64_t F, uint32_t d0,
+                                         uint32_t d1) const {
+        const float* p = w + F;
+        if constexpr (FORM != kOdd) {
+            const f32x2u t =
+                __builtin_nontemporal_load(reinterpret_cast<const f32x2u*>(p + d0));
+            r.v[i][0] = t.x;
+            r.v[i][1] = t.y;
+        } else {
+            r.v[i][0] = p[d0];
+            r.v[i][1] = p[d1];
+        }
+    }
+    __device__ __forceinline__ void pair(Regs& r, int i, int, float& w0, float& w1) const {
+        w0 = r.v[i][0];
+        w1 = r.v[i][1];
+    }
+    __device__ __forceinline__ float at(uint64_t f) const { return w[f]; }
+    static std::string grouped_name(int tm, int wn, int kg) {
+        return tname("split_grouped_kernel", "F32W", tm, wn, kg);
+    }
+};
 
 template <int FORM>
 struct Int8W {
@@ -449,6 +478,66 @@ __global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_product
                                    (b / tiles_m) * S::BN, K, N, ep);
 }
 
+// The grouped products (x [T, K] against `w`'s experts, off [E + 1]): a tile of
+// one expert's rows, the tiles listed column by column so the blocks of an
+// expert meet its weights in one L2.  Offsets in order put expert e's rows at
+// [off[e], min(off[e + 1], T)); offsets that are not (their sum wrapped) give
+// every workgroup a share of the outputs, one lane each, by the reference's
+// e(t) = #{r : off[r + 1] <= t} (grouped.go:48-66).  The matvec form writes 0
+// past the last segment; the matmul form writes only rows that
+// [off[e], min(off[e + 1], T)) covers.
+template <typename W, typename ACT, int TM, int WN, int KG>
+__global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_grouped_kernel(
+    const typename ACT::T* __restrict__ x, W w, const uint32_t* __restrict__ off,
+    float* __restrict__ out, int E, int T, int K, int N, bool matvec) {
+    using S = Shape<ACT, TM, WN, KG>;
+    __shared__ __attribute__((aligned(16))) char lds[S::LDS];
+    const size_t per = (size_t)K * N;
+    const uint64_t lane0 = (uint64_t)blockIdx.x * S::NT + threadIdx.x;
+    const uint64_t lanes = (uint64_t)gridDim.x * S::NT;
+    auto rows_of = [&](int e) {
+        const uint32_t first = off[e], last = min(off[e + 1], (uint32_t)T);
+        return last > first ? (int)(last - first) : 0;
+    };
+    bool in_order = off[0] == 0;
+    int blocks = 0;
+    for (int e = 0; e < E; e++) {
+        in_order = in_order && off[e + 1] >= off[e];
+        blocks += (rows_of(e) + S::BM - 1) / S::BM;
+    }
+    if (!in_order) {
+        for (uint64_t i = lane0; i < (uint64_t)T * N; i += lanes) {
+            const uint32_t t = (uint32_t)(i / N);
+            const int col = (int)(i % N);
+            int e = 0;
+            for (int r = 0; r < E; r++) e += off[r + 1] <= t ? 1 : 0;
+            if (e >= E) {
+                if (matvec) out[i] = 0.0f;
+            } else if (matvec || (t >= off[e] && t < min(off[e + 1], (uint32_t)T))) {
+                out[i] = plain_dot<W, ACT>(x, w.expert(e, per), (size_t)t * K, col, K, N);
+            }
+        }
+        return;
+    }
+    if (matvec)
+        for (uint64_t i = (uint64_t)min(off[E], (uint32_t)T) * N + lane0; i < (uint64_t)T * N;
+             i += lanes)
+            out[i] = 0.0f;
+    const int tiles = blocks * ((N + S::BN - 1) / S::BN);
+    const int per_xcd = (tiles + 7) / 8;
+    const int b = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || b >= tiles) return;
+    int block = b % blocks, e = 0;
+    for (; e < E; e++) {
+        const int n = (rows_of(e) + S::BM - 1) / S::BM;
+        if (block < n) break;
+        block -= n;
+    }
+    split_tile<W, ACT, TM, WN, KG>(lds, x, w.expert(e, per), out, (int)off[e] + block * S::BM,
+                                   (int)min(off[e + 1], (uint32_t)T), (b / blocks) * S::BN, K, N,
+                                   Epilogue{});
+}
+
 // Which tile: the tiles in rounds of the chip, times a K group's stages, times
 // what a stage costs.  The stage costs are measured (us, K = 4096, every CU
 // busy): a wide tile splits its activations for more columns, a narrow one
@@ -505,6 +594,40 @@ hipError_t launch_split(const Device* d, hipStream_t st, const typename ACT::T* 
     }
 }
 
+// The most row blocks of BM rows that T rows of E experts make: each expert
+// that has rows can end in a partial one.
+long long most_blocks(int T, int E, int bm) { return (T + bm - 1) / bm + std::min(T, E); }
+
+template <typename W, typename ACT, int TM, int WN, int KG>
+hipError_t launch_grouped_tile(hipStream_t st, const typename ACT::T* x, W w, const uint32_t* off,
+                               float* out, int E, int T, int K, int N, bool matvec) {
+    using S = Shape<ACT, TM, WN, KG>;
+    const long long wgs = most_blocks(T, E, S::BM) * ((N + S::BN - 1) / S::BN);
+    ACCEL_LAUNCH(W::grouped_name(TM, WN, KG), (split_grouped_kernel<W, ACT, TM, WN, KG>),
+                 dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(S::NT), 0, st, x, w, off, out, E, T, K,
+                 N, matvec);
+    return launch_status();
+}
+
+// Where the rows are is known on the device only: the tile is chosen for rows
+// spread over the experts, half a block left over in each.
+template <typename W, typename ACT>
+hipError_t launch_grouped(const Device* d, hipStream_t st, const typename ACT::T* x, W w,
+                          const uint32_t* off, float* out, int E, int T, int K, int N,
+                          bool matvec) {
+    const int used = std::min(E, T);
+    switch (choose_tile(d, T / 64 + (used + 1) / 2, T / 32 + (used + 1) / 2, K, N)) {
+        case SplitTile::k64x256:
+            return launch_grouped_tile<W, ACT, 2, 4, 2>(st, x, w, off, out, E, T, K, N, matvec);
+        case SplitTile::k64x128:
+            return launch_grouped_tile<W, ACT, 2, 2, 4>(st, x, w, off, out, E, T, K, N, matvec);
+        case SplitTile::k64x64:
+            return launch_grouped_tile<W, ACT, 2, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
+        default:
+            return launch_grouped_tile<W, ACT, 1, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
+    }
+}
+
 template <typename ACT>
 hipError_t launch_split_int8_act(const Device* d, hipStream_t st, const typename ACT::T* a,
                                  const int8_t* q, const uint16_t* s, float* out, int M, int K,
@@ -523,6 +646,19 @@ bool split_product_supported(int M, int K, int N) {
     // workgroups stay below 2^32 lanes at the smallest tile
     return N <= (1 << 24) &&
            (long long)((M + 31) / 32) * ((N + 63) / 64) <= (1ll << 22) && K < (1 << 30);
+}
+
+bool split_grouped_supported(int E, int T, int K, int N) {
+    return N <= (1 << 24) && K < (1 << 30) &&
+           most_blocks(T, E, 32) * ((N + 63) / 64) <= (1ll << 22);
+}
+
+hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,
+                                    const uint32_t* off, float* out, int E, int T, int K, int N,
+                                    bool matvec) {
+    if (N % 2 == 0)
+        return launch_grouped<F32W<kEven>, ActF32>(d, st, x, {w}, off, out, E, T, K, N, matvec);
+    return launch_grouped<F32W<kOdd>, ActF32>(d, st, x, {w}, off, out, E, T, K, N, matvec);
 }
 
 hipError_t launch_split_int8(const Device* d, hipStream_t st, const void* a, bool f16_act,

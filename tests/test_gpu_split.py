@@ -10,7 +10,7 @@ import pytest
 
 import accel_amd
 import oracle
-from accel_amd import F16, F32
+from accel_amd import F16, F32, U32
 from conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -88,3 +88,70 @@ def test_int8_tiny_activations_keep_f32_accuracy(dev):
     got = int8_run(dev, a, q, s, M, K, N)
     assert rel_l2(got.astype(np.float64) * 2.0 ** 115,
                   (a.astype(np.float64) * 2.0 ** 115) @ w.reshape(K, N)) <= F32_TOL
+
+
+def grouped_run(dev, form, x, w, counts, T, K, N):
+    xb, wb = dev.upload(x.reshape(T, K)), dev.upload(w)
+    cb, ob = dev.upload(np.array(counts, np.uint32), U32), dev.alloc((T, N), F32)
+    ob.write(np.full((T, N), 7.0, np.float32))
+    getattr(dev, form)(xb, wb, cb, ob)
+    got = ob.numpy()
+    for b in (xb, wb, cb, ob):
+        b.free()
+    return got
+
+
+# (K, N, counts, T): one row, empty experts, blocks that end in one row, rows
+# past the last segment, N odd and even, K of no whole stage, the four tiles
+GROUPED = [(7, 1, [1], 1), (100, 33, [0, 5, 0, 65], 73), (64, 130, [1, 0, 0, 1], 3),
+           (257, 64, [64, 1, 33, 0], 98), (300, 1022, [129, 3], 140), (1024, 2048, [70, 90, 60], 220),
+           (32, 24000, [200, 300, 140, 1], 641), (130, 1000, [0, 0, 0], 5)]
+
+
+@pytest.mark.parametrize("form", ["GroupedMatVec", "GroupedMatMul"])
+@pytest.mark.parametrize("K,N,counts,T", GROUPED)
+def test_grouped_f32_matches_the_oracle(dev, form, K, N, counts, T):
+    E = len(counts)
+    rng = np.random.default_rng(K * 31 + N)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    w = (rng.standard_normal((E, K, N)) * 0.05).astype(np.float32)
+    got = grouped_run(dev, form, x, w, counts, T, K, N)
+    at = 0
+    for e, c in enumerate(counts):
+        if c:
+            want = x[at:at + c].astype(np.float64) @ w[e].astype(np.float64)
+            assert rel_l2(got[at:at + c], want) <= F32_TOL, e
+        at += c
+    assert np.all(got[at:] == (0 if form == "GroupedMatVec" else 7.0))
+
+
+@pytest.mark.parametrize("form", ["GroupedMatVec", "GroupedMatMul"])
+@pytest.mark.parametrize("counts", [[3, 0xFFFFFFFF, 4, 2], [6, 0xFFFFFFFA, 6], [9, 4]])
+def test_grouped_f32_offsets_that_wrap_or_run_past_the_rows(dev, form, counts):
+    E, T, K, N = len(counts), 8, 96, 70
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    w = rng.standard_normal((E, K, N)).astype(np.float32)
+    got = grouped_run(dev, form, x, w, counts, T, K, N)
+    off = np.concatenate([[0], np.cumsum(np.array(counts, np.uint64)) & 0xFFFFFFFF])
+    for t in range(T):
+        e = int(np.sum(off[1:] <= t))
+        covered = e < E and off[e] <= t < min(off[e + 1], T)
+        if e < E and (covered or form == "GroupedMatVec"):
+            want = x[t].astype(np.float64) @ w[e].astype(np.float64)
+            assert rel_l2(got[t], want) <= F32_TOL, t
+        else:
+            assert np.all(got[t] == (0 if form == "GroupedMatVec" else 7.0)), t
+
+
+def test_grouped_f32_infinite_and_nan_weights_read_as_in_f32(dev):
+    E, T, K, N = 2, 40, 64, 96
+    rng = np.random.default_rng(12)
+    x = np.abs(rng.standard_normal((T, K))).astype(np.float32) + 0.5
+    w = rng.standard_normal((E, K, N)).astype(np.float32)
+    w[0, 3, 5], w[1, 4, 6], w[1, 5, 7] = np.inf, -np.inf, np.nan
+    got = grouped_run(dev, "GroupedMatMul", x, w, [20, 20], T, K, N)
+    assert np.all(got[:20, 5] == np.inf) and np.all(got[20:, 6] == -np.inf)
+    assert np.all(np.isnan(got[20:, 7]))
+    got[:20, 5] = got[20:, 6] = got[20:, 7] = 0
+    assert np.all(np.isfinite(got))
