@@ -2435,8 +2435,11 @@ hipError_t launch_int4_matvec_noalloc(Device* d, hipStream_t st, const float* a,
                                     "resolved when it was opened");
         return hipSuccess;
     }
+    // no scratch, as Int4MatVec routes them
+    if (int4_ragged_rows_supported(a, w.codes, 1, K, N))
+        return launch_int4_ragged_rows(st, a, false, w, out, 1, K, N, Epilogue{});
     if (!int4_decode_f32_supported(1, K, N, w.codes))
-        return launch_int4_generic_f32(st, a, w, out, 1, K, N, Epilogue{});   // no scratch
+        return launch_int4_generic_f32(st, a, w, out, 1, K, N, Epilogue{});
     const int tw = matvec_tile(N);
     if (tw == 512)
         return launch_decode<1, 512, 32>(d, st, a, w, out, K, N, status, Epilogue{}, d->scratch);

@@ -377,6 +377,18 @@ hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float
                                     const uint32_t* off, float* out, int E, int T, int K, int N,
                                     bool matvec);
 
+// The products of int4 matrices of any extents take matrices at least a
+// tile's 64 columns wide and 128 rows deep at 16-byte aligned addresses.
+// Below that a launch is mostly empty and one lane per element is as fast;
+// rows or codes from other addresses keep the kernels that load single
+// elements.
+bool int4_ragged_shape(const void* a, const void* codes, int K, int N);
+// Up to four rows of f32 or bf16 (out then bf16) on a matrix whose width is
+// no multiple of a group: ragged.hip, no workspace.
+bool int4_ragged_rows_supported(const void* a, const void* codes, int M, int K, int N);
+hipError_t launch_int4_ragged_rows(hipStream_t st, const void* a, bool bf16, Int4Planes w,
+                                   void* out, int M, int K, int N, Epilogue ep);
+
 // Device quantizer.
 hipError_t launch_int4_quantize(hipStream_t st, const float* w, int64_t n,
                                 uint32_t* packed, uint16_t* scales, uint16_t* zeros);

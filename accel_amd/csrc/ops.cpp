@@ -138,6 +138,8 @@ enum class Int4Route {
     kDecodeF32,     // M <= 16 f32 rows: the decode kernels
     kGemmF32x3,     // M > 16 f32 rows on the matrix cores, three-term split
     kGemmF32,       // M > 16 f32 rows, fp32 VALU tiles
+    kRaggedF32,     // 1..4 f32 rows, N no multiple of a group
+    kRaggedBf16,    // the same, bf16
     kGenericF32,    // one lane per output element
     kDecodeBf16Row, // one bf16 row: the VALU decode kernel
     kDecodeBf16Rows,// 2..16 bf16 rows: the matrix-core decode kernel
@@ -150,6 +152,10 @@ struct Int4Choice {
     std::string reason;
     std::vector<std::string> rejected;
 };
+
+const char* const kRaggedReason =
+    "1..4 rows on a matrix whose width is no multiple of 128: column strips over all of K, each "
+    "lane's rows eight apart so its code words keep one alignment; no K split, no workspace";
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -191,6 +197,11 @@ Int4Choice choose_int4(int32_t dtype, const void* a, const void* codes, int M, i
                    "they take N a multiple of 128 and 16-byte aligned codes");
         else
             reject("the decode kernels", "they take at most 16 rows a launch");
+        if (int4_ragged_rows_supported(a, codes, M, K, N)) {
+            c.route = Int4Route::kRaggedF32;
+            c.reason = kRaggedReason;
+            return c;
+        }
         if (M > 16 && int4_gemm_f32x3_supported(K, N) && aligned16(a)) {
             c.route = Int4Route::kGemmF32x3;
             c.reason = "more than 16 f32 rows: the bf16 matrix-core tiles to f32 accuracy "
@@ -243,6 +254,12 @@ Int4Choice choose_int4(int32_t dtype, const void* a, const void* codes, int M, i
                    "f32 accumulation); K split when the tiles leave CUs idle";
         return c;
     }
+    if (int4_ragged_rows_supported(a, codes, M, K, N)) {
+        c.route = Int4Route::kRaggedBf16;
+        c.reason = kRaggedReason;
+        reject("the matrix-core tiles", "they take N % 128 == 0");
+        return c;
+    }
     reject("the matrix-core tiles",
            aligned16(a) ? "they take K % 64 == 0, N % 128 == 0, K < 2^22 and N < 2^26"
                         : "the activations are not 16-byte aligned, and the tiles load them "
@@ -267,6 +284,10 @@ hipError_t launch_int4_route(Device* d, hipStream_t st, Int4Route r, const void*
         case Int4Route::kGemmF32x3:
             return launch_int4_gemm_f32x3(d, st, af, p, out, M, K, N, ep, status);
         case Int4Route::kGemmF32: return launch_int4_gemm_f32(d, st, af, p, out, M, K, N, ep);
+        case Int4Route::kRaggedF32:
+            return launch_int4_ragged_rows(st, a, false, p, out, M, K, N, ep);
+        case Int4Route::kRaggedBf16:
+            return launch_int4_ragged_rows(st, a, true, p, out, M, K, N, ep);
         case Int4Route::kGenericF32: return launch_int4_generic_f32(st, af, p, out, M, K, N, ep);
         case Int4Route::kDecodeBf16Row:
             return launch_int4_decode_bf16_row(d, st, ab, p, ob, K, N, status, ep.bias);

@@ -10,7 +10,7 @@ import pytest
 
 import accel_amd
 import oracle
-from accel_amd import F16, F32, U32
+from accel_amd import BF16, F16, F32, U32, workloads
 from conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -155,3 +155,65 @@ def test_grouped_f32_infinite_and_nan_weights_read_as_in_f32(dev):
     assert np.all(np.isnan(got[20:, 7]))
     got[:20, 5] = got[20:, 6] = got[20:, 7] = 0
     assert np.all(np.isfinite(got))
+
+
+def int4_run(dev, a, p, s, z, M, K, N, bf16=False, form="Int4MatMul", bias=None):
+    ab = dev.upload(a, BF16 if bf16 else F32)
+    wd = dev.upload_int4(p, s, z, K * N)
+    ob = dev.alloc((M, N) if a.ndim == 2 else (N,), BF16 if bf16 else F32)
+    bb = dev.upload(bias) if bias is not None else None
+    if form == "Int4Linear":
+        dev.Int4Linear(ab, wd, bb, ob)
+    else:
+        getattr(dev, form)(ab, wd, ob)
+    got, launches = ob.numpy(), dev.last_selection().launches
+    for b in (ab, ob, wd, bb):
+        if b:
+            b.free()
+    return (workloads.bf16_to_f32(got) if bf16 else got), launches
+
+
+def int4_weights(rng, K, N):
+    p, s, z = workloads.fast_int4(K, N, rng)
+    s, z = s.copy(), z.copy()
+    s[1], z[1] = 0, oracle.to_f16(np.array([0.75], np.float32))[0]     # a constant group
+    z[-1] = oracle.to_f16(np.array([-900.0], np.float32))[0]           # far from zero
+    w = oracle.int4_dequantize(p, s, z, K * N).astype(np.float64).reshape(K, N)
+    return p, s, z, w
+
+
+# (K, N): every N mod 8 (the words' alignments), strips that end in one column
+# and in whole, K below, at and past the row phases and their batches
+RAGGED = [(128, 64), (130, 65), (511, 570), (512, 571), (513, 572), (200, 61 + 64), (1000, 1001),
+          (4096, 1004), (129, 4095), (777, 30 * 56), (300, 30 * 56 + 1), (2048, 126)]
+
+
+@pytest.mark.parametrize("K,N", RAGGED)
+def test_int4_matvec_of_any_width_matches_the_oracle(dev, K, N):
+    rng = np.random.Generator(np.random.PCG64(K * 31 + N))
+    p, s, z, w = int4_weights(rng, K, N)
+    for M, bf16 in ((1, False), (1, True), (2, False), (3, True), (4, False)):
+        x = rng.standard_normal((M, K)).astype(np.float32)
+        bits = workloads.bf16_bits(x)
+        want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w
+        if M == 1 and not bf16:
+            got, launches = int4_run(dev, x[0], p, s, z, 1, K, N, form="Int4MatVec")
+            again, _ = int4_run(dev, x[0], p, s, z, 1, K, N, form="Int4MatVecNoAlloc")
+            assert np.array_equal(got, again)
+        else:
+            got, launches = int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16)
+        assert launches[0].startswith("ragged_rows_kernel<"), launches
+        assert rel_l2(got, want if M > 1 or bf16 else want[0]) <= (4e-3 if bf16 else F32_TOL), (M, bf16)
+
+
+def test_int4_matvec_of_any_width_infinities_and_nans(dev):
+    K, N = 300, 203
+    rng = np.random.Generator(np.random.PCG64(9))
+    p, s, z, w = int4_weights(rng, K, N)
+    x = rng.standard_normal(K).astype(np.float32)
+    x[299] = np.inf           # the last row: its words end the planes
+    got, _ = int4_run(dev, x, p, s, z, 1, K, N, form="Int4MatVec")
+    assert np.array_equal(np.isinf(got), w[299] != 0)
+    x[299], x[0] = 1, np.nan
+    got, _ = int4_run(dev, x, p, s, z, 1, K, N, form="Int4MatVec")
+    assert np.all(np.isnan(got))
