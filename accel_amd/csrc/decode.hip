@@ -2437,7 +2437,7 @@ hipError_t launch_int4_matvec_noalloc(Device* d, hipStream_t st, const float* a,
     }
     // no scratch, as Int4MatVec routes them
     if (int4_ragged_rows_supported(a, w.codes, 1, K, N))
-        return launch_int4_ragged_rows(st, a, false, w, out, 1, K, N, Epilogue{});
+        return launch_int4_ragged_rows(d, st, a, false, w, out, 1, K, N, Epilogue{});
     if (!int4_decode_f32_supported(1, K, N, w.codes))
         return launch_int4_generic_f32(st, a, w, out, 1, K, N, Epilogue{});
     const int tw = matvec_tile(N);

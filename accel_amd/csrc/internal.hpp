@@ -386,8 +386,8 @@ bool int4_ragged_shape(const void* a, const void* codes, int K, int N);
 // Up to four rows of f32 or bf16 (out then bf16) on a matrix whose width is
 // no multiple of a group: ragged.hip, no workspace.
 bool int4_ragged_rows_supported(const void* a, const void* codes, int M, int K, int N);
-hipError_t launch_int4_ragged_rows(hipStream_t st, const void* a, bool bf16, Int4Planes w,
-                                   void* out, int M, int K, int N, Epilogue ep);
+hipError_t launch_int4_ragged_rows(const Device* d, hipStream_t st, const void* a, bool bf16,
+                                   Int4Planes w, void* out, int M, int K, int N, Epilogue ep);
 
 // Device quantizer.
 hipError_t launch_int4_quantize(hipStream_t st, const float* w, int64_t n,

@@ -285,9 +285,9 @@ hipError_t launch_int4_route(Device* d, hipStream_t st, Int4Route r, const void*
             return launch_int4_gemm_f32x3(d, st, af, p, out, M, K, N, ep, status);
         case Int4Route::kGemmF32: return launch_int4_gemm_f32(d, st, af, p, out, M, K, N, ep);
         case Int4Route::kRaggedF32:
-            return launch_int4_ragged_rows(st, a, false, p, out, M, K, N, ep);
+            return launch_int4_ragged_rows(d, st, a, false, p, out, M, K, N, ep);
         case Int4Route::kRaggedBf16:
-            return launch_int4_ragged_rows(st, a, true, p, out, M, K, N, ep);
+            return launch_int4_ragged_rows(d, st, a, true, p, out, M, K, N, ep);
         case Int4Route::kGenericF32: return launch_int4_generic_f32(st, af, p, out, M, K, N, ep);
         case Int4Route::kDecodeBf16Row:
             return launch_int4_decode_bf16_row(d, st, ab, p, ob, K, N, status, ep.bias);

@@ -1,10 +1,12 @@
 // Int4MatVec and Int4MatMul of up to four rows on matrices whose width is no
 // multiple of a quantisation group, so groups and code words run across rows.
 //
-// Bound: HBM (the codes), then the VALU: about four instructions a weight.
+// Bound: instruction issue (about 60 a lane's word, 3 cycles each) and, with
+// narrow strips over the whole chip, L2: a row's scale and zero are a 128-byte
+// line each for two bytes.
 //
 // Row k's columns begin at nibble k N, so what a code word means for a column
-// depends on k N mod 8 only.  A workgroup of 512 lanes owns a strip of columns
+// depends on k N mod 8 only.  A workgroup of 1024 lanes owns a strip of columns
 // over all of K; lane (row phase p, l) takes rows p, p + RP, ... with RP a
 // multiple of eight, so its words keep one alignment for the whole of K: word
 // l of the strip, eight fixed columns and, since a word never straddles a
@@ -18,7 +20,7 @@
 // A weight is (q - z) * s as in the per-element kernels, q - z in f32 and the
 // scale folded into the activation; a zero scale reads as z.
 //
-// 4096 x 32004 (one row): 1307 us one lane per element, 81 us here.
+// 4096 x 32004 (one row): 1305 us one lane per element, 39 us here (1.7 TB/s).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,8 +31,8 @@
 namespace accel {
 namespace {
 
-constexpr int kRagThreads = 512;
-constexpr int kRagBatch = 8;   // rows a lane has in flight
+constexpr int kRagThreads = 1024;
+constexpr int kRagBatch = 4;   // rows of a load batch, two batches out at a time
 
 __device__ __forceinline__ float rag_act(float v) { return v; }
 __device__ __forceinline__ float rag_act(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
@@ -65,8 +67,14 @@ __global__ __launch_bounds__(kRagThreads) void ragged_rows_kernel(
     auto shift_of = [&](int phase) { return 8 - (int)(((uint32_t)phase * (uint32_t)(N & 7)) & 7u); };
     const int64_t f0 = (int64_t)p * N + c0 + shift_of(p) - 8 + 8 * l;
     const uint32_t w0 = f0 > 0 ? (uint32_t)(f0 >> 3) : 0u;
-    const uint32_t step = (uint32_t)((uint64_t)RP * (uint64_t)N >> 3);   // words a row step
-    const uint32_t last_word = (uint32_t)(((uint64_t)K * (uint64_t)N + 7) / 8 - 1);
+    // A row step is RP N nibbles, a batch of four a whole number of groups: the
+    // lane's distances from a batch's (uniform) bases never change.
+    const uint64_t step = (uint64_t)RP * (uint64_t)N >> 3;          // words
+    const uint64_t step4 = (uint64_t)RP * (uint64_t)N >> 5;         // groups, four steps
+    static_assert(RP % 32 == 0 && kRagBatch == 4, "four steps are whole groups");
+    uint32_t dw = w0, dx = (uint32_t)p, dg[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) dg[u] = (uint32_t)((w0 + u * step) >> 4);
 
     float acc[M][8], bias[M];
 #pragma unroll
@@ -75,50 +83,102 @@ __global__ __launch_bounds__(kRagThreads) void ragged_rows_kernel(
 #pragma unroll
         for (int j = 0; j < 8; j++) acc[m][j] = 0.0f;
     }
-    const int steps = (K + RP - 1) / RP;
-    for (int i0 = 0; i0 < steps; i0 += kRagBatch) {
+    struct Batch {
         uint32_t q[kRagBatch];
-        uint16_t sb[kRagBatch], zb[kRagBatch];
-        XT xb[kRagBatch][M];
+        uint16_t s[kRagBatch], z[kRagBatch];
+        XT x[kRagBatch][M];
+    };
+    const XT* xp[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) xp[m] = a + (size_t)min(m, rows - 1) * K;
+    // The loads of the steps from i0.  Cached: neighbouring strips share the
+    // 128-byte lines (non-temporal loads fetched them again: 81 against 60 us).
+    auto load = [&](Batch& t, int i0) {
+        const uint32_t* cp = codes + i0 * step;
+        const uint16_t* sp = scales + (i0 >> 2) * step4;
+        const uint16_t* zp = zeros + (i0 >> 2) * step4;
+#pragma unroll
+        for (int u = 0; u < kRagBatch; u++) {
+            t.q[u] = (cp + u * step)[dw];
+            t.s[u] = sp[dg[u]];
+            t.z[u] = zp[dg[u]];
+#pragma unroll
+            for (int m = 0; m < M; m++) t.x[u][m] = (xp[m] + (i0 + u) * RP)[dx];
+        }
+    };
+    // The same for the last steps: rows past the end count nothing, and row
+    // K - 1's windows may run past the planes.
+    auto load_end = [&](Batch& t, int i0) {
+        const uint64_t last_word = ((uint64_t)K * (uint64_t)N + 7) / 8 - 1;
 #pragma unroll
         for (int u = 0; u < kRagBatch; u++) {
             const int k = p + (i0 + u) * RP;
-            // rows past the end load word 0's and count nothing
-            const uint32_t w = k < K ? min(w0 + (uint32_t)(i0 + u) * step, last_word) : 0u;
-            q[u] = __builtin_nontemporal_load(codes + w);
-            sb[u] = scales[w >> 4];
-            zb[u] = zeros[w >> 4];
+            const uint64_t w = k < K ? min(w0 + (i0 + u) * step, last_word) : 0;
+            t.q[u] = codes[w];
+            t.s[u] = k < K ? scales[w >> 4] : (uint16_t)0;
+            t.z[u] = k < K ? zeros[w >> 4] : (uint16_t)0;
 #pragma unroll
-            for (int m = 0; m < M; m++)
-                xb[u][m] = a[(size_t)min(m, rows - 1) * K + min(k, K - 1)];
+            for (int m = 0; m < M; m++) t.x[u][m] = k < K ? xp[m][k] : (XT)0;
         }
+    };
+    auto add = [&](const Batch& t) {
 #pragma unroll
         for (int u = 0; u < kRagBatch; u++) {
-            const bool valid = p + (i0 + u) * RP < K;
-            const float s = valid ? half_bits_to_float(sb[u]) : 0.0f;
-            const float z = valid ? half_bits_to_float(zb[u]) : 0.0f;
-            // nibbles as e4m3 bytes are q 2^-9, exactly
-            const uint32_t even = q[u] & 0x0F0F0F0Fu, odd = (q[u] >> 4) & 0x0F0F0F0Fu;
-            const f32x2 e01 = __builtin_amdgcn_cvt_pk_f32_fp8(even, false);
-            const f32x2 e23 = __builtin_amdgcn_cvt_pk_f32_fp8(even, true);
-            const f32x2 o01 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, false);
-            const f32x2 o23 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, true);
-            const float z9 = z * 0x1p-9f;
-            const float d[8] = {e01.x - z9, o01.x - z9, e01.y - z9, o01.y - z9,
-                                e23.x - z9, o23.x - z9, e23.y - z9, o23.y - z9};
-            const float s9 = s * 512.0f;
+            float s = half_bits_to_float(t.s[u]);
+            const float z = half_bits_to_float(t.z[u]);
+            // a nibble as an e4m3 byte is q 2^-9; the conversion's scale makes
+            // it q, exactly
+            const uint32_t even = t.q[u] & 0x0F0F0F0Fu, odd = (t.q[u] >> 4) & 0x0F0F0F0Fu;
+            const f32x2 e01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, false);
+            const f32x2 e23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, true);
+            const f32x2 o01 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, false);
+            const f32x2 o23 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, true);
+            float x[M], xs[M];
 #pragma unroll
             for (int m = 0; m < M; m++) {
-                const float x = valid ? rag_act(xb[u][m]) : 0.0f;
-                // a zero scale's weights are z; neither side's product may meet
-                // the other's infinite activation with its zero
-                const float xs = s == 0.0f ? 0.0f : x * s9;
-                const float xz = __builtin_fmaf(x, z, bias[m]);
-                bias[m] = s == 0.0f ? xz : bias[m];
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[m][j] = __builtin_fmaf(xs, d[j], acc[m][j]);
+                x[m] = rag_act(t.x[u][m]);
+                xs[m] = x[m] * s;
             }
+            // a zero scale's weights are z, and an infinite activation must not
+            // meet the zero
+            if (__builtin_amdgcn_ballot_w64(s == 0.0f)) {
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    const float xz = __builtin_fmaf(x[m], z, bias[m]);
+                    bias[m] = s == 0.0f ? xz : bias[m];
+                    xs[m] = s == 0.0f ? 0.0f : xs[m];
+                }
+            }
+            const float d[8] = {e01.x - z, o01.x - z, e01.y - z, o01.y - z,
+                                e23.x - z, o23.x - z, e23.y - z, o23.y - z};
+#pragma unroll
+            for (int m = 0; m < M; m++)
+#pragma unroll
+                for (int j = 0; j < 8; j++) acc[m][j] = __builtin_fmaf(xs[m], d[j], acc[m][j]);
         }
+    };
+    // Batches of rows below K - 1, the next one's loads out while one is added
+    // (without a branch between, or the waits drain them); then the rest.
+    const int whole = (K - 1) / (RP * kRagBatch);
+    if (whole > 0) {
+        Batch b0, b1;
+        load(b0, 0);
+        for (int i = 0; i < whole; i += 2) {
+            // marked here: widened to 64 bits outside the loop the distances
+            // would cost an add at every load
+            asm volatile(""
+                         : "+v"(dw), "+v"(dx), "+v"(dg[0]), "+v"(dg[1]), "+v"(dg[2]), "+v"(dg[3]));
+            load(b1, min(i + 1, whole - 1) * kRagBatch);
+            add(b0);
+            if (i + 1 >= whole) break;
+            load(b0, min(i + 2, whole - 1) * kRagBatch);
+            add(b1);
+        }
+    }
+    for (int i0 = whole * kRagBatch; i0 * RP < K; i0 += kRagBatch) {
+        Batch b;
+        load_end(b, i0);
+        add(b);
     }
 
 #pragma unroll
@@ -159,15 +219,31 @@ void launch_ragged(hipStream_t st, const XT* a, Int4Planes w, void* out, int row
                  0, st, a, w.codes, w.scales, w.zeros, out, rows, K, N, ep);
 }
 
-template <typename XT>
-hipError_t launch_ragged_any(hipStream_t st, const XT* a, Int4Planes w, void* out, int M, int K,
-                             int N, Epilogue ep) {
-    if (M == 1)
-        launch_ragged<XT, 1, 8>(st, a, w, out, M, K, N, ep);
-    else if (M == 2)
-        launch_ragged<XT, 2, 8>(st, a, w, out, M, K, N, ep);
+// The strip: narrow strips end sooner (fewer row steps a lane), wide ones share
+// their rows' scale and zero lines among more columns; the narrowest whose
+// strips are one round of the chip, else the widest.  One row, 56 / 120 / 248
+// columns (us): 4096 x 4004 15 / 21 / 38, 4096 x 16001 34 / 23 / 38, 4096 x
+// 32004 63 / 52 / 44.
+template <typename XT, int M>
+void launch_ragged_strip(const Device* d, hipStream_t st, const XT* a, Int4Planes w, void* out,
+                         int rows, int K, int N, Epilogue ep) {
+    if (N <= 56 * (long long)d->cu_count)
+        launch_ragged<XT, M, 8>(st, a, w, out, rows, K, N, ep);
+    else if (N <= 120 * (long long)d->cu_count)
+        launch_ragged<XT, M, 16>(st, a, w, out, rows, K, N, ep);
     else
-        launch_ragged<XT, 4, 8>(st, a, w, out, M, K, N, ep);
+        launch_ragged<XT, M, 32>(st, a, w, out, rows, K, N, ep);
+}
+
+template <typename XT>
+hipError_t launch_ragged_any(const Device* d, hipStream_t st, const XT* a, Int4Planes w, void* out,
+                             int M, int K, int N, Epilogue ep) {
+    if (M == 1)
+        launch_ragged_strip<XT, 1>(d, st, a, w, out, M, K, N, ep);
+    else if (M == 2)
+        launch_ragged_strip<XT, 2>(d, st, a, w, out, M, K, N, ep);
+    else
+        launch_ragged_strip<XT, 4>(d, st, a, w, out, M, K, N, ep);
     return launch_status();
 }
 
@@ -179,18 +255,18 @@ bool int4_ragged_shape(const void* a, const void* codes, int K, int N) {
 }
 
 bool int4_ragged_rows_supported(const void* a, const void* codes, int M, int K, int N) {
-    // word indices are 32-bit, and a row step's words a 32-bit stride
+    // a lane's byte distances, over 64 rows, are 32-bit
     return M >= 1 && M <= 4 && N % 128 != 0 && int4_ragged_shape(a, codes, K, N) &&
-           (uint64_t)K * (uint64_t)N < (1ull << 34) && N < (1 << 28) && K < (1 << 30);
+           N < (1 << 26) && K < (1 << 30);
 }
 
-hipError_t launch_int4_ragged_rows(hipStream_t st, const void* a, bool bf16, Int4Planes w,
+hipError_t launch_int4_ragged_rows(const Device* d, hipStream_t st, const void* a, bool bf16, Int4Planes w,
                                    void* out, int M, int K, int N, Epilogue ep) {
     if (bf16) {
         ep.bf16 = true;
-        return launch_ragged_any(st, static_cast<const uint16_t*>(a), w, out, M, K, N, ep);
+        return launch_ragged_any(d, st, static_cast<const uint16_t*>(a), w, out, M, K, N, ep);
     }
-    return launch_ragged_any(st, static_cast<const float*>(a), w, out, M, K, N, ep);
+    return launch_ragged_any(d, st, static_cast<const float*>(a), w, out, M, K, N, ep);
 }
 
 }  // namespace accel

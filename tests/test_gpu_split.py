@@ -185,7 +185,9 @@ def int4_weights(rng, K, N):
 # (K, N): every N mod 8 (the words' alignments), strips that end in one column
 # and in whole, K below, at and past the row phases and their batches
 RAGGED = [(128, 64), (130, 65), (511, 570), (512, 571), (513, 572), (200, 61 + 64), (1000, 1001),
-          (4096, 1004), (129, 4095), (777, 30 * 56), (300, 30 * 56 + 1), (2048, 126)]
+          (4096, 1004), (129, 4095), (777, 30 * 56), (300, 30 * 56 + 1), (2048, 126),
+          # the strips of 120 and of 248 columns
+          (1000, 14393), (385, 30600), (130, 30723), (700, 31000)]
 
 
 @pytest.mark.parametrize("K,N", RAGGED)
