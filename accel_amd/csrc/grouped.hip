@@ -156,10 +156,12 @@ hipError_t launch_grouped_f32(const Device* d, hipStream_t st, const float* x, c
     return launch_status();
 }
 
-hipError_t launch_int4_grouped_f32(hipStream_t st, const float* x, Int4Planes w,
+hipError_t launch_int4_grouped_f32(const Device* d, hipStream_t st, const float* x, Int4Planes w,
                                    const uint32_t* off, float* out, int E, int T, int K,
                                    int N, bool write_padding) {
     if (T == 0 || N == 0) return hipSuccess;
+    if (split_grouped_supported(E, T, K, N))
+        return launch_split_grouped_int4(d, st, x, w, off, out, E, T, K, N, write_padding);
     dim3 grid((N + 255) / 256, T < 65535 ? T : 65535);
     ACCEL_LAUNCH(tname("grouped_f32_kernel", true), (grouped_f32_kernel<true>), grid,
                  dim3(256), 0, st, x, nullptr, w.codes, w.scales, w.zeros, off, out, E, T, K,

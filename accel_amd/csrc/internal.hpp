@@ -251,7 +251,7 @@ hipError_t launch_segment_offsets(hipStream_t st, const uint32_t* counts,
 hipError_t launch_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,
                               const uint32_t* off, float* out, int E, int T, int K,
                               int N, bool write_padding);
-hipError_t launch_int4_grouped_f32(hipStream_t st, const float* x, Int4Planes w,
+hipError_t launch_int4_grouped_f32(const Device* d, hipStream_t st, const float* x, Int4Planes w,
                                    const uint32_t* off, float* out, int E, int T,
                                    int K, int N, bool write_padding);
 // BASELINE config 1's literal format (32-row groups along K, f32 scale, no
@@ -371,6 +371,13 @@ hipError_t launch_split_int8(const Device* d, hipStream_t st, const void* a, boo
                              const int8_t* quants, const uint16_t* scales, float* out, int M,
                              int K, int N);
 
+// Int4 matrices of any extents the same way: f32 rows, or bf16 rows and result.
+hipError_t launch_split_int4(const Device* d, hipStream_t st, const void* a, bool bf16, Int4Planes w,
+                             void* out, int M, int K, int N, Epilogue ep);
+// Grouped products over int4 experts (K * N % 128 == 0), f32 rows, any offsets.
+hipError_t launch_split_grouped_int4(const Device* d, hipStream_t st, const float* x, Int4Planes w,
+                                     const uint32_t* off, float* out, int E, int T, int K, int N,
+                                     bool matvec);
 // The grouped product over f32 experts the same way, any offsets.
 bool split_grouped_supported(int E, int T, int K, int N);
 hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,

@@ -140,6 +140,8 @@ enum class Int4Route {
     kGemmF32,       // M > 16 f32 rows, fp32 VALU tiles
     kRaggedF32,     // 1..4 f32 rows, N no multiple of a group
     kRaggedBf16,    // the same, bf16
+    kSplitF32,      // more f32 rows of any extents: the tiles of split weights
+    kSplitBf16,     // the same, bf16
     kGenericF32,    // one lane per output element
     kDecodeBf16Row, // one bf16 row: the VALU decode kernel
     kDecodeBf16Rows,// 2..16 bf16 rows: the matrix-core decode kernel
@@ -156,6 +158,13 @@ struct Int4Choice {
 const char* const kRaggedReason =
     "1..4 rows on a matrix whose width is no multiple of 128: column strips over all of K, each "
     "lane's rows eight apart so its code words keep one alignment; no K split, no workspace";
+
+bool split_shape(const void* a, const void* codes, int M, int K, int N) {
+    return int4_ragged_shape(a, codes, K, N) && split_product_supported(M, K, N);
+}
+const char* const kSplitReason =
+    "extents no int4 tile takes: the matrix-core tiles of split weights (each weight dequantised "
+    "in f32 and split into three bf16 terms), K split across the waves of a workgroup";
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -217,6 +226,11 @@ Int4Choice choose_int4(int32_t dtype, const void* a, const void* codes, int M, i
         if (M > 16)
             reject("the f32 matrix-core tiles",
                    "they take K % 64 == 0, N % 128 == 0 and 16-byte aligned rows");
+        if (split_shape(a, codes, M, K, N)) {
+            c.route = Int4Route::kSplitF32;
+            c.reason = kSplitReason;
+            return c;
+        }
         if (M > 16 && aligned128) {
             c.route = Int4Route::kGemmF32;
             c.reason = "more than 16 f32 rows that the matrix-core tiles cannot take: fp32 "
@@ -264,6 +278,11 @@ Int4Choice choose_int4(int32_t dtype, const void* a, const void* codes, int M, i
            aligned16(a) ? "they take K % 64 == 0, N % 128 == 0, K < 2^22 and N < 2^26"
                         : "the activations are not 16-byte aligned, and the tiles load them "
                           "16 bytes at a time");
+    if (split_shape(a, codes, M, K, N)) {
+        c.route = Int4Route::kSplitBf16;
+        c.reason = kSplitReason;
+        return c;
+    }
     c.route = Int4Route::kGenericBf16;
     c.reason = "no tiled kernel takes this shape or alignment: one lane per output element, "
                "decoding with the flat index (correct everywhere, not a speed path)";
@@ -288,6 +307,10 @@ hipError_t launch_int4_route(Device* d, hipStream_t st, Int4Route r, const void*
             return launch_int4_ragged_rows(d, st, a, false, p, out, M, K, N, ep);
         case Int4Route::kRaggedBf16:
             return launch_int4_ragged_rows(d, st, a, true, p, out, M, K, N, ep);
+        case Int4Route::kSplitF32:
+            return launch_split_int4(d, st, a, false, p, out, M, K, N, ep);
+        case Int4Route::kSplitBf16:
+            return launch_split_int4(d, st, a, true, p, out, M, K, N, ep);
         case Int4Route::kGenericF32: return launch_int4_generic_f32(st, af, p, out, M, K, N, ep);
         case Int4Route::kDecodeBf16Row:
             return launch_int4_decode_bf16_row(d, st, ab, p, ob, K, N, status, ep.bias);
@@ -956,7 +979,8 @@ int run_grouped_int4(const char* op, int dev, void* stream, const accel_tensor_t
                  "each expert's 128-row blocks";
         rejected = "the decode kernels: they take at most 1024 f32 rows";
     } else if (f32) {
-        reason = "no tiled kernel takes this shape or alignment: one lane per (row, column)";
+        reason = "f32 rows no int4 tile takes: the matrix-core tiles of split weights (rows and "
+                 "dequantised weights in three bf16 terms each), any extents and offsets";
         rejected = "the f32 matrix-core tiles: they take K % 64 == 0, N % 128 == 0 and "
                    "16-byte aligned rows; the decode kernels: at most 1024 rows";
     } else {
@@ -983,7 +1007,7 @@ int run_grouped_int4(const char* op, int dev, void* stream, const accel_tensor_t
             e = launch_zero_tail_f32(st, seg, static_cast<float*>(out->data), (int)experts,
                                      (int)T, (int)N);
     } else if (f32) {
-        e = launch_int4_grouped_f32(st, static_cast<const float*>(x->data), p, off,
+        e = launch_int4_grouped_f32(d, st, static_cast<const float*>(x->data), p, off,
                                     static_cast<float*>(out->data), (int)experts, (int)T,
                                     (int)K, (int)N, matvec);
     } else {

@@ -1,12 +1,15 @@
-// Products to f32 accuracy on the bf16 matrix cores for weights of the int8
-// format and for the grouped products' plain f32 experts.  Every weight is dequantised exactly as the per-element kernels do
+// Products to f32 accuracy on the bf16 matrix cores for weights that are not
+// whole 128-column int4 groups: the int8 format, the grouped products' plain
+// f32 experts, and int4 matrices of any extents (their groups then run across
+// rows).  Every weight is dequantised exactly as the per-element kernels do
 // it, in f32, and both sides are split into bf16 terms (bf16split.hpp):
 //     f32 rows x weights:  3 x 3 terms, the six products above 2^-27 kept
 //     f16 rows:            2 x 3 terms (an f16 is two terms exactly), five
+//     bf16 rows:           1 x 3 terms, three
 // summed in f32 by v_mfma_f32_32x32x16_bf16, the small products first.  What
 // is dropped (2^-26 of a product) is below the rounding of one f32 sum.
 //
-// Bound: the matrix cores, at five or six times the product's flops; for few
+// Bound: the matrix cores, at three to six times the product's flops; for few
 // rows the weight bytes.
 //
 // A workgroup of eight waves computes a BM x BN tile, BN = 64 WN columns: wave
@@ -56,6 +59,12 @@ struct ActF16 {
     static constexpr int kTerms = 2;
     static __device__ __forceinline__ float value(T v) { return half_bits_to_float(v); }
 };
+struct ActBf16 {
+    typedef uint16_t T;
+    static constexpr int kTerms = 1;
+    static __device__ __forceinline__ float value(T v) { return __uint_as_float((uint32_t)v << 16); }
+};
+
 // ---- weight sources ---------------------------------------------------------
 //
 // A lane's unit is eight rows of two columns.  load(r, i, F, d0, d1) fetches
@@ -132,6 +141,63 @@ struct Int8W {
     }
     __device__ __forceinline__ float at(uint64_t f) const {
         return (float)q[f] * half_bits_to_float(s[f >> 5]);
+    }
+};
+
+// The int4 format with groups of 128 flat weights that may run across rows:
+// (code - z) * s, or z where the scale is zero.
+template <int FORM>
+struct Int4W {
+    const uint8_t* c;      // two codes a byte, low nibble first
+    const uint16_t* s;
+    const uint16_t* z;
+    // an experts' stacked planes: whole groups each
+    __device__ __forceinline__ Int4W expert(int e, size_t per) const {
+        return {c + e * (per >> 1), s + e * (per >> 7), z + e * (per >> 7)};
+    }
+    struct Regs { uint32_t c[8], s[8], z[8], c1[8], s1[8], z1[8]; };   // the last three: odd N only
+    __device__ __forceinline__ void load(Regs& r, int i, uint64_t F, uint32_t d0,
+                                         uint32_t d1) const {
+        const uint8_t* cp = c + (F >> 1);
+        const uint16_t* sp = s + (F >> 7);
+        const uint16_t* zp = z + (F >> 7);
+        const uint32_t fg = FORM == kRows ? 0u : (uint32_t)F & 127u;
+        if constexpr (FORM != kOdd) {
+            r.c[i] = cp[d0 >> 1];
+            r.s[i] = sp[(fg + d0) >> 7];
+            r.z[i] = zp[(fg + d0) >> 7];
+        } else {
+            const uint32_t fc = (uint32_t)F & 1u;
+            r.c[i] = cp[(fc + d0) >> 1];
+            r.c1[i] = cp[(fc + d1) >> 1];
+            r.s[i] = sp[(fg + d0) >> 7];
+            r.z[i] = zp[(fg + d0) >> 7];
+            r.s1[i] = sp[(fg + d1) >> 7];
+            r.z1[i] = zp[(fg + d1) >> 7];
+        }
+    }
+    static __device__ __forceinline__ float weight(uint32_t code, uint32_t sb, uint32_t zb) {
+        const float sv = half_bits_to_float((uint16_t)sb), zv = half_bits_to_float((uint16_t)zb);
+        return sv == 0.0f ? zv : ((float)code - zv) * sv;
+    }
+    // flat: the first column's flat index, for which nibble is whose
+    __device__ __forceinline__ void pair(Regs& r, int i, int flat, float& w0, float& w1) const {
+        asm volatile("" : "+v"(r.c[i]), "+v"(r.s[i]), "+v"(r.z[i]));
+        if constexpr (FORM != kOdd) {
+            w0 = weight(r.c[i] & 15u, r.s[i], r.z[i]);
+            w1 = weight(r.c[i] >> 4, r.s[i], r.z[i]);
+        } else {
+            asm volatile("" : "+v"(r.c1[i]), "+v"(r.s1[i]), "+v"(r.z1[i]));
+            const int sh = 4 * (flat & 1);
+            w0 = weight((r.c[i] >> sh) & 15u, r.s[i], r.z[i]);
+            w1 = weight((r.c1[i] >> (4 - sh)) & 15u, r.s1[i], r.z1[i]);
+        }
+    }
+    __device__ __forceinline__ float at(uint64_t f) const {
+        return weight((c[f >> 1] >> (4 * (f & 1))) & 15u, s[f >> 7], z[f >> 7]);
+    }
+    static std::string grouped_name(int tm, int wn, int kg) {
+        return tname("split_grouped_kernel", "Int4W", tm, wn, kg);
     }
 };
 
@@ -577,16 +643,23 @@ hipError_t launch_split_tile(hipStream_t st, const typename ACT::T* a, W w, void
     using S = Shape<ACT, TM, WN, KG>;
     const long long tiles =
         (long long)((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN);
-    hipLaunchKernelGGL((split_product_kernel<W, ACT, TM, WN, KG>),
-                       dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(S::NT), 0, st, a, w, out, M, K,
-                       N, ep);
-    return hipGetLastError();
+    ACCEL_LAUNCH(tname("split_product_kernel", TM, WN, KG) + grid_note(tiles, 1),
+                 (split_product_kernel<W, ACT, TM, WN, KG>),
+                 dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(S::NT), 0, st, a, w, out, M, K, N, ep);
+    return launch_status();
 }
+
+// Odd int4 widths load six words a row of a unit: with 64 rows' accumulators
+// beside them a wave would spill, so they take the 32-row tile.
+template <typename W> constexpr bool kNarrowOnly = false;
+template <> constexpr bool kNarrowOnly<Int4W<kOdd>> = true;
 
 template <typename W, typename ACT>
 hipError_t launch_split(const Device* d, hipStream_t st, const typename ACT::T* a, W w, void* out,
                         int M, int K, int N, Epilogue ep) {
-    switch (choose_tile(d, (M + 63) / 64, (M + 31) / 32, K, N)) {
+    if constexpr (kNarrowOnly<W>)
+        return launch_split_tile<W, ACT, 1, 1, 8>(st, a, w, out, M, K, N, ep);
+    else switch (choose_tile(d, (M + 63) / 64, (M + 31) / 32, K, N)) {
         case SplitTile::k64x256: return launch_split_tile<W, ACT, 2, 4, 2>(st, a, w, out, M, K, N, ep);
         case SplitTile::k64x128: return launch_split_tile<W, ACT, 2, 2, 4>(st, a, w, out, M, K, N, ep);
         case SplitTile::k64x64: return launch_split_tile<W, ACT, 2, 1, 8>(st, a, w, out, M, K, N, ep);
@@ -616,7 +689,9 @@ hipError_t launch_grouped(const Device* d, hipStream_t st, const typename ACT::T
                           const uint32_t* off, float* out, int E, int T, int K, int N,
                           bool matvec) {
     const int used = std::min(E, T);
-    switch (choose_tile(d, T / 64 + (used + 1) / 2, T / 32 + (used + 1) / 2, K, N)) {
+    if constexpr (kNarrowOnly<W>)
+        return launch_grouped_tile<W, ACT, 1, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
+    else switch (choose_tile(d, T / 64 + (used + 1) / 2, T / 32 + (used + 1) / 2, K, N)) {
         case SplitTile::k64x256:
             return launch_grouped_tile<W, ACT, 2, 4, 2>(st, x, w, off, out, E, T, K, N, matvec);
         case SplitTile::k64x128:
@@ -659,6 +734,37 @@ hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float
     if (N % 2 == 0)
         return launch_grouped<F32W<kEven>, ActF32>(d, st, x, {w}, off, out, E, T, K, N, matvec);
     return launch_grouped<F32W<kOdd>, ActF32>(d, st, x, {w}, off, out, E, T, K, N, matvec);
+}
+
+hipError_t launch_split_int4(const Device* d, hipStream_t st, const void* a, bool bf16, Int4Planes w,
+                             void* out, int M, int K, int N, Epilogue ep) {
+    const uint8_t* c = reinterpret_cast<const uint8_t*>(w.codes);
+    auto run = [&](auto act) {
+        using ACT = decltype(act);
+        const auto* x = static_cast<const typename ACT::T*>(a);
+        if (N % 128 == 0)
+            return launch_split<Int4W<kRows>, ACT>(d, st, x, {c, w.scales, w.zeros}, out, M, K, N, ep);
+        if (N % 2 == 0)
+            return launch_split<Int4W<kEven>, ACT>(d, st, x, {c, w.scales, w.zeros}, out, M, K, N, ep);
+        return launch_split<Int4W<kOdd>, ACT>(d, st, x, {c, w.scales, w.zeros}, out, M, K, N, ep);
+    };
+    if (!bf16) return run(ActF32{});
+    ep.bf16 = true;
+    return run(ActBf16{});
+}
+
+hipError_t launch_split_grouped_int4(const Device* d, hipStream_t st, const float* x, Int4Planes w,
+                                     const uint32_t* off, float* out, int E, int T, int K, int N,
+                                     bool matvec) {
+    const uint8_t* c = reinterpret_cast<const uint8_t*>(w.codes);
+    if (N % 128 == 0)
+        return launch_grouped<Int4W<kRows>, ActF32>(d, st, x, {c, w.scales, w.zeros}, off, out, E, T,
+                                                    K, N, matvec);
+    if (N % 2 == 0)
+        return launch_grouped<Int4W<kEven>, ActF32>(d, st, x, {c, w.scales, w.zeros}, off, out, E, T,
+                                                    K, N, matvec);
+    return launch_grouped<Int4W<kOdd>, ActF32>(d, st, x, {c, w.scales, w.zeros}, off, out, E, T, K, N,
+                                               matvec);
 }
 
 hipError_t launch_split_int8(const Device* d, hipStream_t st, const void* a, bool f16_act,

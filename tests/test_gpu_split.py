@@ -219,3 +219,64 @@ def test_int4_matvec_of_any_width_infinities_and_nans(dev):
     x[299], x[0] = 1, np.nan
     got, _ = int4_run(dev, x, p, s, z, 1, K, N, form="Int4MatVec")
     assert np.all(np.isnan(got))
+
+
+# (M, K, N): N odd, even and whole groups (there K % 64 != 0 keeps the int4
+# tiles off), K of no whole stage, one row past the few-rows kernel, and the
+# four tiles
+INT4 = [(5, 128, 65), (6, 129, 64), (33, 200, 1001), (17, 511, 130), (64, 1000, 999),
+        (100, 4100, 4004), (40, 136, 384), (70, 2090, 256), (513, 260, 8190), (300, 1026, 4098),
+        (65, 130, 16391)]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M,K,N", INT4)
+def test_int4_rows_of_any_extents_match_the_oracle(dev, M, K, N, bf16):
+    rng = np.random.Generator(np.random.PCG64(M * 31 + K * 17 + N))
+    p, s, z, w = int4_weights(rng, K, N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    bits = workloads.bf16_bits(x)
+    got, launches = int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16, "Int4Linear", bias)
+    assert launches[0].startswith("split_product_kernel<"), launches
+    want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w + bias
+    # bf16: one rounding of the result (2^-9 at most, 2^-9 / sqrt(3) in the norm)
+    assert rel_l2(got, want) <= (2.0 ** -9 if bf16 else F32_TOL)
+
+
+def test_int4_rows_of_any_extents_infinities(dev):
+    M, K, N = 20, 300, 203
+    rng = np.random.Generator(np.random.PCG64(10))
+    p, s, z, w = int4_weights(rng, K, N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[2, 299], x[3, 0] = -np.inf, np.nan
+    got, _ = int4_run(dev, x, p, s, z, M, K, N)
+    assert np.array_equal(got[2] == -np.inf, w[299] > 0)
+    assert np.array_equal(got[2] == np.inf, w[299] < 0)
+    assert np.all(np.isnan(got[3])) and np.all(np.isfinite(np.delete(got, (2, 3), 0)))
+
+
+@pytest.mark.parametrize("form", ["Int4GroupedMatVec", "Int4GroupedMatMul"])
+@pytest.mark.parametrize("K,N,counts,T", [(128, 33, [3, 0, 40], 45), (256, 130, [1, 70], 71),
+                                          (160, 4, [2, 3], 6), (384, 1002, [100, 0xFFFFFFFF, 30], 120)])
+def test_int4_grouped_of_any_width_matches_the_oracle(dev, form, K, N, counts, T):
+    E = len(counts)
+    rng = np.random.Generator(np.random.PCG64(K + N))
+    p, s, z, w = int4_weights(rng, E * K, N)
+    w = w.reshape(E, K, N)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    xb, wd = dev.upload(x), dev.upload_int4(p, s, z, E * K * N)
+    cb, ob = dev.upload(np.array(counts, np.uint32), U32), dev.alloc((T, N), F32)
+    ob.write(np.full((T, N), 7.0, np.float32))
+    getattr(dev, form)(xb, wd, E, cb, ob)
+    got, launches = ob.numpy(), dev.last_selection().launches
+    for b in (xb, wd, cb, ob):
+        b.free()
+    assert any(k.startswith("split_grouped_kernel<Int4W") for k in launches), launches
+    off = np.concatenate([[0], np.cumsum(np.array(counts, np.uint64)) & 0xFFFFFFFF])
+    for t in range(T):
+        e = int(np.sum(off[1:] <= t))
+        if e < E and (form == "Int4GroupedMatVec" or off[e] <= t < min(off[e + 1], T)):
+            assert rel_l2(got[t], x[t].astype(np.float64) @ w[e]) <= F32_TOL, t
+        else:
+            assert np.all(got[t] == (0 if form == "Int4GroupedMatVec" else 7.0)), t

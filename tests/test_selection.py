@@ -209,3 +209,23 @@ def test_prepared_rows_need_even_k_and_aligned_rows():
         A.select(2, 1001, 4096, A.F32, a=ALIGNED, op="Int4MatMulPrepared")
     with pytest.raises(A.Refused, match="K even"):
         A.select(2, 4096, 4096, A.F32, a=ALIGNED + 4, op="Int4MatMulPrepared")
+
+
+@pytest.mark.parametrize("M,K,N,dtype,name", [
+    (1, 4096, 32004, A.F32, "ragged_rows_kernel<float, 1, 32>"),
+    (1, 128, 64, A.BF16, "ragged_rows_kernel<unsigned short, 1, 8>"),
+    (3, 1000, 15001, A.F32, "ragged_rows_kernel<float, 4, 16>"),
+    (5, 1000, 1001, A.F32, "split_product_kernel<1, 1, 8>"),
+    (100, 4100, 4004, A.F32, "split_product_kernel<1, 1, 8>"),
+    (512, 4100, 4096, A.BF16, "split_product_kernel<2, 2, 4>"),
+    (17, 127, 128, A.F32, "int4_gemm_f32_kernel"),
+    (1, 128, 63, A.F32, "int4_generic_f32_kernel"),
+])
+def test_matrices_of_any_extents(M, K, N, dtype, name):
+    """Widths that are no multiple of a group and depths no tile takes: up to
+    four rows on the column strips, more on the tiles of split weights; below
+    64 columns or 128 rows, or off 16-byte alignment, as before."""
+    sel = A.select(M, K, N, dtype, a=ALIGNED, codes=ALIGNED)
+    assert _names(sel) == [name], sel
+    off = A.select(M, K, N, dtype, a=ALIGNED + 4, codes=ALIGNED)
+    assert not any(k.startswith(("ragged", "split")) for k in _names(off)), off
