@@ -280,3 +280,29 @@ def test_int4_grouped_of_any_width_matches_the_oracle(dev, form, K, N, counts, T
             assert rel_l2(got[t], x[t].astype(np.float64) @ w[e]) <= F32_TOL, t
         else:
             assert np.all(got[t] == (0 if form == "Int4GroupedMatVec" else 7.0)), t
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 16384 + 1920, 3 * 2048 + 128 * 5 + 77])
+def test_packer_waves_of_sixteen_groups_are_bit_exact(dev, n):
+    """Whole waves beside single groups, and waves that leave the fast path:
+    a NaN or infinity anywhere, a -0.0 minimum, constant groups, ranges whose
+    f16 scale is zero, subnormal or infinite."""
+    rng = np.random.default_rng(n)
+    base = (rng.standard_normal(n) * 0.02).astype(np.float32)
+    odd = base.copy()
+    odd[-128:] = 0.0
+    odd[: 128] = np.abs(odd[: 128])
+    odd[5] = -0.0
+    odd[300] = np.nan
+    odd[1023] = np.inf
+    scales = np.repeat(10.0 ** rng.integers(-12, 30, n // 128 + 1), 128)[:n]
+    for w in (base, odd, np.maximum(base, 0), (base * scales).astype(np.float32),
+              np.full(n, -3.25, np.float32), np.zeros(n, np.float32)):
+        wb = dev.upload(w)
+        pb, sb = dev.alloc(((n + 7) // 8,), U32), dev.alloc(((n + 127) // 128,), F16)
+        zb = dev.alloc(((n + 127) // 128,), F16)
+        dev.int4_quantize(wb, n, pb, sb, zb)
+        for got, want in zip((pb, sb, zb), oracle.int4_quantize(w)):
+            assert np.array_equal(got.numpy(), want)
+        for b in (wb, pb, sb, zb):
+            b.free()
