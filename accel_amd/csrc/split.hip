@@ -12,8 +12,8 @@
 // Bound: the matrix cores, at three to six times the product's flops; for few
 // rows the weight bytes.
 //
-// A workgroup of eight waves computes a BM x BN tile, BN = 64 WN columns: wave
-// (wn, g) owns 64 columns and the K group g of KG.  The weights need no LDS:
+// A workgroup of eight waves (sixteen for the narrow tile, 32 columns) computes
+// a BM x BN tile, BN = 64 WN columns: wave (wn, g) owns 64 columns and the K group g of KG.  The weights need no LDS:
 // a lane loads eight consecutive k of two adjacent columns, which after the
 // split are exactly its operands of two n-tiles (MFMA column c of n-tile j is
 // tile column 2 c + j).  The activations are shared by the waves of a K group
@@ -73,32 +73,36 @@ struct ActBf16 {
 // weights, dequantised as the per-element kernels do it.  FORM says how rows
 // lie: kOdd, any N; kEven, N even, so a pair is adjacent and in one
 // quantisation block, one load; kRows, N a multiple of the block, so a row's
-// scales start at a whole block.
+// scales start at a whole block.  kOne is a lane of one column, any N: the
+// narrow tile's.
 // F and the row's base stay in scalar registers.
-enum { kOdd, kEven, kRows };
+enum { kOdd, kEven, kRows, kOne };
+constexpr bool paired(int form) { return form == kEven || form == kRows; }
 
 // Plain f32 weights (the grouped products' experts, [K, N] each).
 template <int FORM>
 struct F32W {
+    using One = F32W<kOne>;
+    One one() const { return {w}; }
     const float* w;
     __device__ __forceinline__ F32W expert(int e, size_t per) const { return {w + e * per}; }
     struct Regs { float v[8][2]; };
     __device__ __forceinline__ void load(Regs& r, int i, uint64_t F, uint32_t d0,
                                          uint32_t d1) const {
         const float* p = w + F;
-        if constexpr (FORM != kOdd) {
+        if constexpr (paired(FORM)) {
             const f32x2u t =
                 __builtin_nontemporal_load(reinterpret_cast<const f32x2u*>(p + d0));
             r.v[i][0] = t.x;
             r.v[i][1] = t.y;
         } else {
             r.v[i][0] = p[d0];
-            r.v[i][1] = p[d1];
+            if constexpr (FORM == kOdd) r.v[i][1] = p[d1];
         }
     }
     __device__ __forceinline__ void pair(Regs& r, int i, int, float& w0, float& w1) const {
         w0 = r.v[i][0];
-        w1 = r.v[i][1];
+        if constexpr (FORM != kOne) w1 = r.v[i][1];
     }
     __device__ __forceinline__ float at(uint64_t f) const { return w[f]; }
     static std::string grouped_name(int tm, int wn, int kg) {
@@ -108,6 +112,8 @@ struct F32W {
 
 template <int FORM>
 struct Int8W {
+    using One = Int8W<kOne>;
+    One one() const { return {q, s}; }
     const int8_t* q;
     const uint16_t* s;
     struct Regs { uint32_t q[8], s[8], q1[8], s1[8]; };   // q1, s1: odd N only
@@ -116,14 +122,16 @@ struct Int8W {
         const int8_t* qp = q + F;
         const uint16_t* sp = s + (F >> 5);
         const uint32_t fs = (uint32_t)F & 31u;
-        if constexpr (FORM != kOdd) {
+        if constexpr (paired(FORM)) {
             r.q[i] = *reinterpret_cast<const u16u*>(qp + d0);
             r.s[i] = FORM == kRows ? sp[d0 >> 5] : sp[(fs + d0) >> 5];
         } else {
             r.q[i] = (uint8_t)qp[d0];
-            r.q1[i] = (uint8_t)qp[d1];
             r.s[i] = sp[(fs + d0) >> 5];
-            r.s1[i] = sp[(fs + d1) >> 5];
+            if constexpr (FORM == kOdd) {
+                r.q1[i] = (uint8_t)qp[d1];
+                r.s1[i] = sp[(fs + d1) >> 5];
+            }
         }
     }
     __device__ __forceinline__ void pair(Regs& r, int i, int, float& w0, float& w1) const {
@@ -132,9 +140,9 @@ struct Int8W {
         asm volatile("" : "+v"(r.q[i]), "+v"(r.s[i]));
         const float s0 = half_bits_to_float((uint16_t)r.s[i]);
         w0 = (float)(int8_t)r.q[i] * s0;
-        if constexpr (FORM != kOdd) {
+        if constexpr (paired(FORM)) {
             w1 = (float)(int8_t)(r.q[i] >> 8) * s0;
-        } else {
+        } else if constexpr (FORM == kOdd) {
             asm volatile("" : "+v"(r.q1[i]), "+v"(r.s1[i]));
             w1 = (float)(int8_t)r.q1[i] * half_bits_to_float((uint16_t)r.s1[i]);
         }
@@ -148,6 +156,8 @@ struct Int8W {
 // (code - z) * s, or z where the scale is zero.
 template <int FORM>
 struct Int4W {
+    using One = Int4W<kOne>;
+    One one() const { return {c, s, z}; }
     const uint8_t* c;      // two codes a byte, low nibble first
     const uint16_t* s;
     const uint16_t* z;
@@ -162,18 +172,20 @@ struct Int4W {
         const uint16_t* sp = s + (F >> 7);
         const uint16_t* zp = z + (F >> 7);
         const uint32_t fg = FORM == kRows ? 0u : (uint32_t)F & 127u;
-        if constexpr (FORM != kOdd) {
+        if constexpr (paired(FORM)) {
             r.c[i] = cp[d0 >> 1];
             r.s[i] = sp[(fg + d0) >> 7];
             r.z[i] = zp[(fg + d0) >> 7];
         } else {
             const uint32_t fc = (uint32_t)F & 1u;
             r.c[i] = cp[(fc + d0) >> 1];
-            r.c1[i] = cp[(fc + d1) >> 1];
             r.s[i] = sp[(fg + d0) >> 7];
             r.z[i] = zp[(fg + d0) >> 7];
-            r.s1[i] = sp[(fg + d1) >> 7];
-            r.z1[i] = zp[(fg + d1) >> 7];
+            if constexpr (FORM == kOdd) {
+                r.c1[i] = cp[(fc + d1) >> 1];
+                r.s1[i] = sp[(fg + d1) >> 7];
+                r.z1[i] = zp[(fg + d1) >> 7];
+            }
         }
     }
     static __device__ __forceinline__ float weight(uint32_t code, uint32_t sb, uint32_t zb) {
@@ -183,13 +195,14 @@ struct Int4W {
     // flat: the first column's flat index, for which nibble is whose
     __device__ __forceinline__ void pair(Regs& r, int i, int flat, float& w0, float& w1) const {
         asm volatile("" : "+v"(r.c[i]), "+v"(r.s[i]), "+v"(r.z[i]));
-        if constexpr (FORM != kOdd) {
+        if constexpr (paired(FORM)) {
             w0 = weight(r.c[i] & 15u, r.s[i], r.z[i]);
             w1 = weight(r.c[i] >> 4, r.s[i], r.z[i]);
         } else {
-            asm volatile("" : "+v"(r.c1[i]), "+v"(r.s1[i]), "+v"(r.z1[i]));
             const int sh = 4 * (flat & 1);
             w0 = weight((r.c[i] >> sh) & 15u, r.s[i], r.z[i]);
+            if constexpr (FORM == kOne) return;
+            asm volatile("" : "+v"(r.c1[i]), "+v"(r.s1[i]), "+v"(r.z1[i]));
             w1 = weight((r.c1[i] >> (4 - sh)) & 15u, r.s1[i], r.z1[i]);
         }
     }
@@ -205,7 +218,8 @@ struct Int4W {
 
 template <typename ACT, int TM, int WN, int KG>
 struct Shape {
-    static constexpr int BM = 32 * TM, BN = 64 * WN;
+    static constexpr int TN = KG == 16 ? 1 : 2;        // columns a lane
+    static constexpr int BM = 32 * TM, BN = 32 * TN * WN;
     static constexpr int TG = 64 * WN;                 // lanes of a K group
     static constexpr int NT = KG * TG;
     static constexpr int NA = ACT::kTerms;
@@ -238,7 +252,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
                                            const W& w, void* __restrict__ out, int m0, int m_end,
                                            int n0, int K, int N, const Epilogue& ep) {
     using S = Shape<ACT, TM, WN, KG>;
-    constexpr int NA = S::NA, BM = S::BM, BN = S::BN, TG = S::TG;
+    constexpr int NA = S::NA, BM = S::BM, BN = S::BN, TG = S::TG, TN = S::TN;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave / WN, wn = wave % WN;
@@ -261,13 +275,13 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
         ap[u] = a + (size_t)min(m0 + a_row + u * (TG / 4), m_end - 1) * K + 8 * a_oct;
     // the lane's columns as flat distances from the tile's first; columns past
     // the edge are clamped copies, never stored
-    const int cp = 2 * (32 * wn + c32);
-    const uint32_t c0 = N % 2 == 0 ? min(cp, N - 2 - n0) : min(cp, N - 1 - n0);
+    const int cp = TN * (32 * wn + c32);
+    const uint32_t c0 = TN == 2 && N % 2 == 0 ? min(cp, N - 2 - n0) : min(cp, N - 1 - n0);
     const uint32_t c1 = min(cp + 1, N - 1 - n0);
 
     typename ACT::T ra[S::AU][8];
     typename W::Regs rb[2];
-    bf16x8 bf[2][3][2];      // [half stage][term][column]
+    bf16x8 bf[2][3][TN];     // [half stage][term][column]
     uint32_t ta[4][NA];      // a unit of A being split
     float wv[2][2];          // two rows of B being split: [row][column]
 
@@ -335,18 +349,18 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
         }
     };
 
-    f32x16 acc[TM][2];
+    f32x16 acc[TM][TN];
 #pragma unroll
     for (int t = 0; t < TM; t++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[t][j][r] = 0.0f;
 
     // Half h of the stage in `buf`: its products, terms x + y <= 2 with the
     // smallest first, and between them `chunks` pieces of other work.
     constexpr int kSums = NA == 3 ? 6 : NA == 2 ? 5 : 3;   // kept term pairs
-    constexpr int kMfma = kSums * TM * 2;
+    constexpr int kMfma = kSums * TM * TN;
     auto multiply = [&](int buf, int h, auto chunks, auto&& other) {
         constexpr int C = decltype(chunks)::value;
         bf16x8 af[NA][TM];
@@ -365,7 +379,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
 #pragma unroll
                 for (int t = 0; t < TM; t++)
 #pragma unroll
-                    for (int j = 0; j < 2; j++) {
+                    for (int j = 0; j < TN; j++) {
                         acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                             af[x][t], bf[h][sum - x][j], acc[t][j], 0, 0, 0);
                         if (C > 0) {
@@ -385,7 +399,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
             const int p = c / 3;
             if (c % 3 == 0) dequant_b(h, p, of);
             if (c % 3 == 1) split_b(h, p, 0);
-            if (c % 3 == 2) split_b(h, p, 1);
+            if (TN == 2 && c % 3 == 2) split_b(h, p, 1);
         } else {
             load_b(h, c - 12, load);
         }
@@ -480,7 +494,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
             for (int r = 0; r < 16; r++) {
                 const int rl = t * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+                for (int j = 0; j < TN; j++)
                     if (rl < rows && cp + j < cols) {
                         const float v = acc[t][j][r];
                         odd = __builtin_fmaf(v, 0.0f, odd);
@@ -495,8 +509,11 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int rl = t * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
-                *reinterpret_cast<f32x2*>(sums + (g * BM + rl) * BN + cp) =
-                    (f32x2){acc[t][0][r], acc[t][1][r]};
+                float* at = sums + (g * BM + rl) * BN + cp;
+                if constexpr (TN == 2)
+                    *reinterpret_cast<f32x2*>(at) = (f32x2){acc[t][0][r], acc[t][TN - 1][r]};
+                else
+                    *at = acc[t][0][r];
             }
         __syncthreads();
 #pragma unroll 4
@@ -527,7 +544,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
 }
 
 template <typename W, typename ACT, int TM, int WN, int KG>
-__global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_product_kernel(
+__global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), (KG == 16 ? 4 : 2)) void split_product_kernel(
     const typename ACT::T* __restrict__ a, W w, void* __restrict__ out, int M, int K, int N,
     Epilogue ep) {
     using S = Shape<ACT, TM, WN, KG>;
@@ -553,7 +570,7 @@ __global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_product
 // past the last segment; the matmul form writes only rows that
 // [off[e], min(off[e + 1], T)) covers.
 template <typename W, typename ACT, int TM, int WN, int KG>
-__global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_grouped_kernel(
+__global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), (KG == 16 ? 4 : 2)) void split_grouped_kernel(
     const typename ACT::T* __restrict__ x, W w, const uint32_t* __restrict__ off,
     float* __restrict__ out, int E, int T, int K, int N, bool matvec) {
     using S = Shape<ACT, TM, WN, KG>;
@@ -607,10 +624,11 @@ __global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), 2) void split_grouped
 // Which tile: the tiles in rounds of the chip, times a K group's stages, times
 // what a stage costs.  The stage costs are measured (us, K = 4096, every CU
 // busy): a wide tile splits its activations for more columns, a narrow one
-// fills the chip with fewer rows and columns.  512 x 4096 x 4096 int8 (us):
-// 64 x 256 tiles 142, 64 x 128 90, 64 x 64 120, 32 x 64 157; 2048 rows 334,
-// 363, 437, 560; 128 rows 136, 76, 49, 39.
-enum class SplitTile { k64x256, k64x128, k64x64, k32x64 };
+// fills the chip with fewer rows and columns.  int8, K = N = 4096 (us), tiles
+// of 64 x 256, 64 x 128, 64 x 64, 32 x 64 and 32 x 32: 512 rows 151, 96, 131,
+// 163, 229; 128 rows 134, 73, 46, 37, 54; 32 rows 132, 73, 46, 35, 27; and 33 x
+// 4864 x 352 157, 86, 52, 40, 30.
+enum class SplitTile { k64x256, k64x128, k64x64, k32x64, k32x32 };
 
 SplitTile choose_tile(const Device* d, long long rows_blocks64, long long rows_blocks32, int K,
                       int N) {
@@ -622,7 +640,8 @@ SplitTile choose_tile(const Device* d, long long rows_blocks64, long long rows_b
     } const kTiles[] = {{SplitTile::k64x256, rows_blocks64, 256, 2, 2.6},
                         {SplitTile::k64x128, rows_blocks64, 128, 4, 2.85},
                         {SplitTile::k64x64, rows_blocks64, 64, 8, 3.5},
-                        {SplitTile::k32x64, rows_blocks32, 64, 8, 2.4}};
+                        {SplitTile::k32x64, rows_blocks32, 64, 8, 2.4},
+                        {SplitTile::k32x32, rows_blocks32, 32, 16, 3.1}};
     SplitTile best = SplitTile::k32x64;
     double best_us = 1e30;
     for (const auto& k : kTiles) {
@@ -657,13 +676,18 @@ template <> constexpr bool kNarrowOnly<Int4W<kOdd>> = true;
 template <typename W, typename ACT>
 hipError_t launch_split(const Device* d, hipStream_t st, const typename ACT::T* a, W w, void* out,
                         int M, int K, int N, Epilogue ep) {
+    const SplitTile tile = choose_tile(d, (M + 63) / 64, (M + 31) / 32, K, N);
     if constexpr (kNarrowOnly<W>)
-        return launch_split_tile<W, ACT, 1, 1, 8>(st, a, w, out, M, K, N, ep);
-    else switch (choose_tile(d, (M + 63) / 64, (M + 31) / 32, K, N)) {
+        return tile == SplitTile::k32x32
+                   ? launch_split_tile<typename W::One, ACT, 1, 1, 16>(st, a, w.one(), out, M, K, N, ep)
+                   : launch_split_tile<W, ACT, 1, 1, 8>(st, a, w, out, M, K, N, ep);
+    else switch (tile) {
         case SplitTile::k64x256: return launch_split_tile<W, ACT, 2, 4, 2>(st, a, w, out, M, K, N, ep);
         case SplitTile::k64x128: return launch_split_tile<W, ACT, 2, 2, 4>(st, a, w, out, M, K, N, ep);
         case SplitTile::k64x64: return launch_split_tile<W, ACT, 2, 1, 8>(st, a, w, out, M, K, N, ep);
-        default: return launch_split_tile<W, ACT, 1, 1, 8>(st, a, w, out, M, K, N, ep);
+        case SplitTile::k32x64: return launch_split_tile<W, ACT, 1, 1, 8>(st, a, w, out, M, K, N, ep);
+        default:
+            return launch_split_tile<typename W::One, ACT, 1, 1, 16>(st, a, w.one(), out, M, K, N, ep);
     }
 }
 
@@ -689,17 +713,24 @@ hipError_t launch_grouped(const Device* d, hipStream_t st, const typename ACT::T
                           const uint32_t* off, float* out, int E, int T, int K, int N,
                           bool matvec) {
     const int used = std::min(E, T);
+    const SplitTile tile = choose_tile(d, T / 64 + (used + 1) / 2, T / 32 + (used + 1) / 2, K, N);
     if constexpr (kNarrowOnly<W>)
-        return launch_grouped_tile<W, ACT, 1, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
-    else switch (choose_tile(d, T / 64 + (used + 1) / 2, T / 32 + (used + 1) / 2, K, N)) {
+        return tile == SplitTile::k32x32
+                   ? launch_grouped_tile<typename W::One, ACT, 1, 1, 16>(st, x, w.one(), off, out, E, T,
+                                                                         K, N, matvec)
+                   : launch_grouped_tile<W, ACT, 1, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
+    else switch (tile) {
         case SplitTile::k64x256:
             return launch_grouped_tile<W, ACT, 2, 4, 2>(st, x, w, off, out, E, T, K, N, matvec);
         case SplitTile::k64x128:
             return launch_grouped_tile<W, ACT, 2, 2, 4>(st, x, w, off, out, E, T, K, N, matvec);
         case SplitTile::k64x64:
             return launch_grouped_tile<W, ACT, 2, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
-        default:
+        case SplitTile::k32x64:
             return launch_grouped_tile<W, ACT, 1, 1, 8>(st, x, w, off, out, E, T, K, N, matvec);
+        default:
+            return launch_grouped_tile<typename W::One, ACT, 1, 1, 16>(st, x, w.one(), off, out, E, T,
+                                                                       K, N, matvec);
     }
 }
 
@@ -718,14 +749,14 @@ hipError_t launch_split_int8_act(const Device* d, hipStream_t st, const typename
 
 bool split_product_supported(int M, int K, int N) {
     // a lane's 32-bit distances span sixteen rows; the grid's 512-lane
-    // workgroups stay below 2^32 lanes at the smallest tile
+    // or 1024-lane workgroups stay below 2^32 lanes at the smallest tile
     return N <= (1 << 24) &&
-           (long long)((M + 31) / 32) * ((N + 63) / 64) <= (1ll << 22) && K < (1 << 30);
+           (long long)((M + 31) / 32) * ((N + 31) / 32) <= (1ll << 21) && K < (1 << 30);
 }
 
 bool split_grouped_supported(int E, int T, int K, int N) {
     return N <= (1 << 24) && K < (1 << 30) &&
-           most_blocks(T, E, 32) * ((N + 63) / 64) <= (1ll << 22);
+           most_blocks(T, E, 32) * ((N + 31) / 32) <= (1ll << 21);
 }
 
 hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float* x, const float* w,

@@ -215,7 +215,7 @@ def test_prepared_rows_need_even_k_and_aligned_rows():
     (1, 4096, 32004, A.F32, "ragged_rows_kernel<float, 1, 32>"),
     (1, 128, 64, A.BF16, "ragged_rows_kernel<unsigned short, 1, 8>"),
     (3, 1000, 15001, A.F32, "ragged_rows_kernel<float, 4, 16>"),
-    (5, 1000, 1001, A.F32, "split_product_kernel<1, 1, 8>"),
+    (5, 1000, 1001, A.F32, "split_product_kernel<1, 1, 16>"),
     (100, 4100, 4004, A.F32, "split_product_kernel<1, 1, 8>"),
     (512, 4100, 4096, A.BF16, "split_product_kernel<2, 2, 4>"),
     (17, 127, 128, A.F32, "int4_gemm_f32_kernel"),
