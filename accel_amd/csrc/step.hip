@@ -112,58 +112,81 @@ __global__ __launch_bounds__(kRowLanes) void rmsnorm_kernel(const float* __restr
     }
 }
 
-// Rows up to kLdsWidth wide: the whole row and the gain go to LDS with
-// 16-byte loads from all 256 lanes at once (one memory round trip), lanes
-// 0..127 then form the reference's 128 strided partials from LDS in the
-// reference's order, and every lane writes its share of the output.
-constexpr int kLdsThreads = 256;
+// Rows up to kLdsWidth wide, a workgroup a row: every lane loads its 16-byte
+// pieces of the row and of the gain at once and keeps them in registers (one
+// memory round trip, and the sums do not wait for the gain); the row also goes
+// to LDS, where lanes 0..127 form the reference's 128 strided partials in its
+// order; the halving tree runs within waves but for its first step.  Bound by
+// latency at decode sizes: the launch, the round trip, 32 dependent additions
+// a partial (4096 wide) and the f64 root and reciprocal.  A lane holds one
+// piece up to 4096 wide, so lanes follow the width: 2048 rows of 1024 on 1024
+// lanes 7.0 us, on 256 4.6.  From 256 lanes with row and gain through LDS: 512 x
+// 4096 5.5 -> 4.7 us, 2048 x 4096 15.3 -> 13.6, 1 x 14336 8.6 -> 4.5; a batch-8
+// decoder layer with two of them 85.7 -> 83.5.
 constexpr int kLdsWidth = 16384;
 
-__global__ __launch_bounds__(kLdsThreads) void rmsnorm_lds_kernel(const float* __restrict__ x,
-                                                                  const float* __restrict__ w,
-                                                                  float* __restrict__ out,
-                                                                  int width, float eps) {
+template <int LANES, int NV>
+__global__ __launch_bounds__(LANES) void rmsnorm_lds_kernel(const float* __restrict__ x,
+                                                            const float* __restrict__ w,
+                                                            float* __restrict__ out, int width,
+                                                            float eps) {
 #pragma clang fp contract(off)
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    float* xs = smem;            // [width]
-    float* ws = smem + width;    // [width]
+    extern __shared__ __attribute__((aligned(16))) float xs[];   // [width]
     __shared__ float sh[kRowLanes];
+    __shared__ float total;
     const int t = threadIdx.x;
     const float* xr = x + (size_t)blockIdx.x * width;
     float* orow = out + (size_t)blockIdx.x * width;
     const int w4 = width / 4;    // width % 4 == 0 and 16-byte rows on this path
-    for (int i = t; i < w4; i += kLdsThreads) {
-        reinterpret_cast<f32x4*>(xs)[i] = reinterpret_cast<const f32x4*>(xr)[i];
-        reinterpret_cast<f32x4*>(ws)[i] = reinterpret_cast<const f32x4*>(w)[i];
-    }
+    f32x4 v[NV], g[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if (t + i * LANES < w4) v[i] = reinterpret_cast<const f32x4*>(xr)[t + i * LANES];
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if (t + i * LANES < w4) g[i] = reinterpret_cast<const f32x4*>(w)[t + i * LANES];
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if (t + i * LANES < w4) reinterpret_cast<f32x4*>(xs)[t + i * LANES] = v[i];
     __syncthreads();
     if (t < kRowLanes) {
         float acc = 0.0f;
+#pragma unroll 8
         for (int i = t; i < width; i += kRowLanes) {
-            const float v = xs[i];
-            const float sq = v * v;
+            const float e = xs[i];
+            const float sq = e * e;
             acc = acc + sq;
         }
         sh[t] = acc;
     }
     __syncthreads();
-    for (int stride = kRowLanes / 2; stride > 0; stride /= 2) {
-        if (t < stride) sh[t] = sh[t] + sh[t + stride];
-        __syncthreads();
-    }
-    const float mean = sh[0] / (float)width;
-    const float scale = (float)(1.0 / sqrt((double)(mean + eps)));
-    for (int i = t; i < w4; i += kLdsThreads) {
-        const f32x4 v = reinterpret_cast<const f32x4*>(xs)[i];
-        const f32x4 g = reinterpret_cast<const f32x4*>(ws)[i];
-        f32x4 r;
+    if (t < 64) {
+        float s = sh[t] + sh[t + 64];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float p = v[j] * scale;
-            r[j] = p * g[j];
-        }
-        reinterpret_cast<f32x4*>(orow)[i] = r;
+        for (int stride = 32; stride > 0; stride /= 2) s = s + __shfl_down(s, stride, 64);
+        if (t == 0) total = s;
     }
+    __syncthreads();
+    const float mean = total / (float)width;
+    const float scale = (float)(1.0 / sqrt((double)(mean + eps)));
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if (t + i * LANES < w4) {
+            f32x4 r;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float p = v[i][j] * scale;
+                r[j] = p * g[i][j];
+            }
+            reinterpret_cast<f32x4*>(orow)[t + i * LANES] = r;
+        }
+}
+
+template <int LANES, int NV>
+void launch_rmsnorm_lds(hipStream_t st, const float* x, const float* w, float* out, int rows,
+                        int width, float eps) {
+    hipLaunchKernelGGL((rmsnorm_lds_kernel<LANES, NV>), dim3(rows), dim3(LANES),
+                       (size_t)width * sizeof(float), st, x, w, out, width, eps);
 }
 
 }  // namespace
@@ -185,8 +208,16 @@ hipError_t launch_rmsnorm(hipStream_t st, const float* x, const float* w, float*
     const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
                            reinterpret_cast<uintptr_t>(out)) & 15) == 0;
     if (aligned && width % 4 == 0 && width <= kLdsWidth) {
-        hipLaunchKernelGGL(rmsnorm_lds_kernel, dim3(rows), dim3(kLdsThreads),
-                           (size_t)2 * width * sizeof(float), st, x, w, out, width, eps);
+        if (width <= 1024)
+            launch_rmsnorm_lds<256, 1>(st, x, w, out, rows, width, eps);
+        else if (width <= 2048)
+            launch_rmsnorm_lds<512, 1>(st, x, w, out, rows, width, eps);
+        else if (width <= 4096)
+            launch_rmsnorm_lds<1024, 1>(st, x, w, out, rows, width, eps);
+        else if (width <= 8192)
+            launch_rmsnorm_lds<1024, 2>(st, x, w, out, rows, width, eps);
+        else
+            launch_rmsnorm_lds<1024, 4>(st, x, w, out, rows, width, eps);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(kRowLanes), 0, st, x, w, out, width,

@@ -146,3 +146,9 @@ def test_records_dispatch(dev):
     assert rel_l2(mvb.numpy(), oracle.matvec_f32_f16(av, wv, K, N)) <= F32_TOL
     for t in (ab, bb, ob, xb, gb, rb, avb, wvb, mvb):
         t.free()
+
+
+@pytest.mark.parametrize("rows,width", [(2, 4), (2, 1028), (2, 2048), (2, 2052), (3, 4100),
+                                        (2, 8192), (1, 8196), (2, 16384), (1, 16388)])
+def test_rmsnorm_at_the_edges_of_its_lane_counts_is_bit_exact(dev, rows, width):
+    test_rmsnorm_is_bit_exact(dev, rows, width)
