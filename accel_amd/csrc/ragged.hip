@@ -250,7 +250,7 @@ hipError_t launch_ragged_any(const Device* d, hipStream_t st, const XT* a, Int4P
 }  // namespace
 
 bool int4_ragged_shape(const void* a, const void* codes, int K, int N) {
-    return K >= 128 && N >= 64 &&
+    return K >= (N % 128 ? 32 : 128) && N >= 64 &&
            ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(codes)) & 15) == 0;
 }
 

@@ -190,7 +190,9 @@ struct Int4W {
     }
     static __device__ __forceinline__ float weight(uint32_t code, uint32_t sb, uint32_t zb) {
         const float sv = half_bits_to_float((uint16_t)sb), zv = half_bits_to_float((uint16_t)zb);
-        return sv == 0.0f ? zv : ((float)code - zv) * sv;
+        // the selection is a row's, not a weight's: the product is zero there
+        // (or NaN for an infinite zero point, and then computed again)
+        return __builtin_fmaf((float)code - zv, sv, sv == 0.0f ? zv : 0.0f);
     }
     // flat: the first column's flat index, for which nibble is whose
     __device__ __forceinline__ void pair(Regs& r, int i, int flat, float& w0, float& w1) const {
@@ -207,7 +209,9 @@ struct Int4W {
         }
     }
     __device__ __forceinline__ float at(uint64_t f) const {
-        return weight((c[f >> 1] >> (4 * (f & 1))) & 15u, s[f >> 7], z[f >> 7]);
+        const float sv = half_bits_to_float(s[f >> 7]), zv = half_bits_to_float(z[f >> 7]);
+        const uint32_t code = (c[f >> 1] >> (4 * (f & 1))) & 15u;
+        return sv == 0.0f ? zv : ((float)code - zv) * sv;
     }
     static std::string grouped_name(int tm, int wn, int kg) {
         return tname("split_grouped_kernel", "Int4W", tm, wn, kg);

@@ -184,7 +184,7 @@ def int4_weights(rng, K, N):
 
 # (K, N): every N mod 8 (the words' alignments), strips that end in one column
 # and in whole, K below, at and past the row phases and their batches
-RAGGED = [(128, 64), (130, 65), (511, 570), (512, 571), (513, 572), (200, 61 + 64), (1000, 1001),
+RAGGED = [(32, 65), (33, 70), (128, 66), (130, 65), (511, 570), (512, 571), (513, 572), (200, 61 + 64), (1000, 1001),
           (4096, 1004), (129, 4095), (777, 30 * 56), (300, 30 * 56 + 1), (2048, 126),
           # the strips of 120 and of 248 columns
           (1000, 14393), (385, 30600), (130, 30723), (700, 31000)]
@@ -224,7 +224,7 @@ def test_int4_matvec_of_any_width_infinities_and_nans(dev):
 # (M, K, N): N odd, even and whole groups (there K % 64 != 0 keeps the int4
 # tiles off), K of no whole stage, one row past the few-rows kernel, and the
 # four tiles
-INT4 = [(5, 128, 65), (6, 129, 64), (33, 200, 1001), (17, 511, 130), (64, 1000, 999),
+INT4 = [(5, 128, 65), (6, 129, 64), (9, 32, 66), (40, 47, 333), (33, 200, 1001), (17, 511, 130), (64, 1000, 999),
         (100, 4100, 4004), (40, 136, 384), (70, 2090, 256), (513, 260, 8190), (300, 1026, 4098),
         (65, 130, 16391)]
 

@@ -220,11 +220,14 @@ def test_prepared_rows_need_even_k_and_aligned_rows():
     (512, 4100, 4096, A.BF16, "split_product_kernel<2, 2, 4>"),
     (17, 127, 128, A.F32, "int4_gemm_f32_kernel"),
     (1, 128, 63, A.F32, "int4_generic_f32_kernel"),
+    (1, 31, 100, A.F32, "int4_generic_f32_kernel"),
+    (9, 32, 66, A.BF16, "split_product_kernel<1, 1, 8>"),
 ])
 def test_matrices_of_any_extents(M, K, N, dtype, name):
     """Widths that are no multiple of a group and depths no tile takes: up to
     four rows on the column strips, more on the tiles of split weights; below
-    64 columns or 128 rows, or off 16-byte alignment, as before."""
+    64 columns or 32 rows (128 where N is whole groups), or off 16-byte
+    alignment, as before."""
     sel = A.select(M, K, N, dtype, a=ALIGNED, codes=ALIGNED)
     assert _names(sel) == [name], sel
     off = A.select(M, K, N, dtype, a=ALIGNED + 4, codes=ALIGNED)
