@@ -10,7 +10,8 @@
 // over all of K; lane (row phase p, l) takes rows p, p + RP, ... with RP a
 // multiple of eight, so its words keep one alignment for the whole of K: word
 // l of the strip, eight fixed columns and, since a word never straddles a
-// group, one scale and zero per row.  No shifts, no selections, no second word.
+// group, one scale and zero per row.  No shifts, no second word; a zero scale is
+// one selection a row.
 // The windows of the phases differ by up to seven columns; a strip is eight
 // columns narrower than its LPR words so that every phase covers all of it,
 // and the sums meet by column in LDS, waves first (the phases of one lane are
