@@ -19,7 +19,8 @@
 // K is never split across workgroups: no workspace, no hand-off.
 //
 // A weight is (q - z) * s as in the per-element kernels, q - z in f32 and the
-// scale folded into the activation; a zero scale reads as z.
+// scale folded into the activation; a zero scale reads as z.  A sum that comes
+// out infinite or NaN is computed again by the per-element loop.
 //
 // 4096 x 32004 (one row): 1305 us one lane per element, 39 us here (1.7 TB/s).
 #include <hip/hip_runtime.h>
@@ -37,6 +38,23 @@ constexpr int kRagBatch = 4;   // rows of a load batch, two batches out at a tim
 
 __device__ __forceinline__ float rag_act(float v) { return v; }
 __device__ __forceinline__ float rag_act(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
+
+// The per-element kernels' loop for one output.
+template <typename XT>
+__device__ __attribute__((noinline)) float ragged_dot(const XT* x, const uint32_t* codes,
+                                                      const uint16_t* scales,
+                                                      const uint16_t* zeros, int col, int K,
+                                                      int N) {
+    float acc = 0.0f;
+    for (int k = 0; k < K; k++) {
+        const uint64_t f = (uint64_t)k * N + col;
+        const uint32_t code = (codes[f >> 3] >> (4 * (f & 7))) & 15u;
+        const float s = half_bits_to_float(scales[f >> 7]);
+        const float z = half_bits_to_float(zeros[f >> 7]);
+        acc = __builtin_fmaf(rag_act(x[k]), s == 0.0f ? z : ((float)code - z) * s, acc);
+    }
+    return acc;
+}
 
 // XT: f32 or bf16 bits.  M: rows computed (clamped copies past `rows`).
 template <typename XT, int M, int LPR>
@@ -205,6 +223,10 @@ __global__ __launch_bounds__(kRagThreads) void ragged_rows_kernel(
             float v = 0.0f;
 #pragma unroll
             for (int ph = 0; ph < 8; ph++) v += fin[ph][c + 8];
+            // an activation times its scale may overflow where its products
+            // with the weights do not
+            if ((__float_as_uint(v) & 0x7f800000u) == 0x7f800000u)
+                v = ragged_dot(xp[m], codes, scales, zeros, c0 + c, K, N);
             store_out(out, (size_t)m * N + c0 + c, c0 + c, v, ep);
         }
     }

@@ -221,6 +221,26 @@ def test_int4_matvec_of_any_width_infinities_and_nans(dev):
     assert np.all(np.isnan(got))
 
 
+@pytest.mark.parametrize("M", [1, 3])
+def test_int4_rows_whose_scaled_activation_overflows_stay_finite(dev, M):
+    # 1e36 x 4096 overflows, but where the code is the zero point the weight is 0
+    K, N = 300, 203
+    rng = np.random.Generator(np.random.PCG64(10))
+    p, s, z, _ = int4_weights(rng, K, N)
+    s[8], z[8] = oracle.to_f16(np.array([4096.0, 8.0], np.float32))   # of row 5: columns 9..136
+    w = oracle.int4_dequantize(p, s, z, K * N).astype(np.float64).reshape(K, N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[M - 1, 5] = 1e36
+    got, launches = int4_run(dev, x, p, s, z, M, K, N)
+    assert launches[0].startswith("ragged_rows_kernel<"), launches
+    want = x.astype(np.float64) @ w
+    over = np.abs(want) > 3.5e38
+    assert over.any() and np.sum(w[5, 9:137] == 0) > 0
+    assert np.array_equal(np.isinf(got), over)
+    bound = K * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w))   # of K f32 roundings
+    assert np.all(np.abs(got - want)[~over] <= bound[~over])
+
+
 # (M, K, N): N odd, even and whole groups (there K % 64 != 0 keeps the int4
 # tiles off), K of no whole stage, one row past the few-rows kernel, and the
 # four tiles
