@@ -8,6 +8,15 @@
 //     bf16 rows:           1 x 3 terms, three
 // summed in f32 by v_mfma_f32_32x32x16_bf16, the small products first.  What
 // is dropped (2^-26 of a product) is below the rounding of one f32 sum.
+// bf16 ends where f32 does, at 2^-126, and a third term is 2^-17 of its value:
+// so f32 values are split as 2^24 times themselves (exact), which puts even
+// their last bit, 2^-149, among bf16's normal numbers, and the sums are scaled
+// back (exact but for results that are subnormal).  Without it relative errors
+// were 4e-5 at 2^-120 and 2e-3 at 2^-126.  It costs a multiplication an f32
+// value (us without / with, one card): int8 512 x 4096 x 4096 97.9 / 98.7, 256
+// rows of 8 f32 experts of 2048 x 4096 73.9 / 74.6, int4 100 x 4100 x 4004
+// 48.0 / 49.1.  Operands from 2^104 on (sums from 2^80 with f32 experts) leave
+// the range and are computed again as below.
 //
 // Bound: the matrix cores, at three to six times the product's flops; for few
 // rows the weight bytes.
@@ -23,9 +32,9 @@
 // still fills it, without a workspace, so products on different streams share
 // nothing and a capture needs no earlier call.
 //
-// A product that overflowed or met an infinity or a NaN (any of which the
-// split turns into a non-finite sum) is computed again by the per-element
-// loop, so such values read as they do there.
+// A product that overflowed, scaled or not, or met an infinity or a NaN (any
+// of which the split turns into a non-finite sum) is computed again by the
+// per-element loop, so such values read as they do there.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,22 +55,26 @@ typedef uint16_t u16x8u __attribute__((ext_vector_type(8), aligned(2)));
 typedef uint16_t u16u __attribute__((aligned(1)));
 
 constexpr int KS = 32;   // k of a stage
+constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;   // f32 values in the split
 
 // ---- activations ----------------------------------------------------------
 
 struct ActF32 {
     typedef float T;
     static constexpr int kTerms = 3;
+    static constexpr float kScale = kUp, kUnscale = kDown;   // of the values split
     static __device__ __forceinline__ float value(T v) { return v; }
 };
 struct ActF16 {
     typedef uint16_t T;
     static constexpr int kTerms = 2;
+    static constexpr float kScale = 1.0f, kUnscale = 1.0f;
     static __device__ __forceinline__ float value(T v) { return half_bits_to_float(v); }
 };
 struct ActBf16 {
     typedef uint16_t T;
-    static constexpr int kTerms = 1;
+    static constexpr int kTerms = 1;   // itself: not split
+    static constexpr float kUnscale = 1.0f;
     static __device__ __forceinline__ float value(T v) { return __uint_as_float((uint32_t)v << 16); }
 };
 
@@ -70,7 +83,8 @@ struct ActBf16 {
 // A lane's unit is eight rows of two columns.  load(r, i, F, d0, d1) fetches
 // row i of a unit: F is the flat index of the (uniform) row and tile column,
 // d0 and d1 the lane's distances to its two columns.  pair() gives row i's
-// weights, dequantised as the per-element kernels do it.  FORM says how rows
+// weights to split, 1 / kUnscale times what at() gives: dequantised as the
+// per-element kernels do it.  FORM says how rows
 // lie: kOdd, any N; kEven, N even, so a pair is adjacent and in one
 // quantisation block, one load; kRows, N a multiple of the block, so a row's
 // scales start at a whole block.  kOne is a lane of one column, any N: the
@@ -84,6 +98,7 @@ template <int FORM>
 struct F32W {
     using One = F32W<kOne>;
     One one() const { return {w}; }
+    static constexpr float kUnscale = kDown;
     const float* w;
     __device__ __forceinline__ F32W expert(int e, size_t per) const { return {w + e * per}; }
     struct Regs { float v[8][2]; };
@@ -101,8 +116,8 @@ struct F32W {
         }
     }
     __device__ __forceinline__ void pair(Regs& r, int i, int, float& w0, float& w1) const {
-        w0 = r.v[i][0];
-        if constexpr (FORM != kOne) w1 = r.v[i][1];
+        w0 = r.v[i][0] * kUp;
+        if constexpr (FORM != kOne) w1 = r.v[i][1] * kUp;
     }
     __device__ __forceinline__ float at(uint64_t f) const { return w[f]; }
     static std::string grouped_name(int tm, int wn, int kg) {
@@ -114,6 +129,7 @@ template <int FORM>
 struct Int8W {
     using One = Int8W<kOne>;
     One one() const { return {q, s}; }
+    static constexpr float kUnscale = 1.0f;   // a weight is 0 or at least 2^-24
     const int8_t* q;
     const uint16_t* s;
     struct Regs { uint32_t q[8], s[8], q1[8], s1[8]; };   // q1, s1: odd N only
@@ -158,6 +174,7 @@ template <int FORM>
 struct Int4W {
     using One = Int4W<kOne>;
     One one() const { return {c, s, z}; }
+    static constexpr float kUnscale = 1.0f;   // a weight is 0 or at least 2^-48
     const uint8_t* c;      // two codes a byte, low nibble first
     const uint16_t* s;
     const uint16_t* z;
@@ -316,7 +333,8 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
         if constexpr (NA == 1)
             ta[p][0] = (uint32_t)ra[u][2 * p] | ((uint32_t)ra[u][2 * p + 1] << 16);
         else
-            split_terms<NA>(ACT::value(ra[u][2 * p]), ACT::value(ra[u][2 * p + 1]), ta[p]);
+            split_terms<NA>(ACT::value(ra[u][2 * p]) * ACT::kScale,
+                            ACT::value(ra[u][2 * p + 1]) * ACT::kScale, ta[p]);
     };
     auto write_a = [&](int u, int buf) {
         const int row = a_row + u * (TG / 4);
@@ -489,6 +507,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
     }
 
     // out, through LDS in K group order when there are several
+    constexpr float kBack = ACT::kUnscale * W::kUnscale;
     float odd = 0.0f;   // becomes NaN when a sum is not finite
     const int rows = min(BM, m_end - m0), cols = min(BN, N - n0);
     if constexpr (KG == 1) {
@@ -500,7 +519,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
 #pragma unroll
                 for (int j = 0; j < TN; j++)
                     if (rl < rows && cp + j < cols) {
-                        const float v = acc[t][j][r];
+                        const float v = acc[t][j][r] * kBack;
                         odd = __builtin_fmaf(v, 0.0f, odd);
                         store_out(out, (size_t)(m0 + rl) * N + n0 + cp + j, n0 + cp + j, v, ep);
                     }
@@ -526,6 +545,7 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
             float v = sums[i];
 #pragma unroll
             for (int q = 1; q < KG; q++) v += sums[q * BM * BN + i];
+            v *= kBack;
             if (rl < rows && cl < cols) {
                 odd = __builtin_fmaf(v, 0.0f, odd);
                 store_out(out, (size_t)(m0 + rl) * N + n0 + cl, n0 + cl, v, ep);

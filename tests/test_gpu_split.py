@@ -50,6 +50,28 @@ def test_int8_matches_the_oracle(dev, M, K, N, f16):
     assert rel_l2(got, x @ w.reshape(K, N)) <= F32_TOL
 
 
+# Activations near the ends of the f32 range, weights of ordinary size: the
+# smallest normals, subnormals (17 bits left near 2^-132) and values whose bf16
+# terms' products pass the largest f32 on the way.  An f32 sum of such products
+# rounds at 2^-150, far below the bound.
+ENDS = [-132, -126, -120, -115, 100, 112]
+
+
+def scaled_l2(got, want, e):
+    return rel_l2(np.ldexp(got.astype(np.float64), -e), np.ldexp(want, -e))
+
+
+@pytest.mark.parametrize("e", ENDS)
+@pytest.mark.parametrize("M,K,N", [(16, 256, 128), (40, 300, 203)])
+def test_int8_rows_at_the_ends_of_the_f32_range(dev, M, K, N, e):
+    rng = np.random.default_rng(M + 200 + e)
+    a = np.ldexp(rng.standard_normal((M, K)), e).astype(np.float32)
+    q, s = oracle.int8_quantize(rng.standard_normal(K * N).astype(np.float32))
+    w = q.astype(np.float64) * oracle.f16_to_f32(s).astype(np.float64)[np.arange(K * N) // 32]
+    got = int8_run(dev, a, q, s, M, K, N)
+    assert scaled_l2(got, a.astype(np.float64) @ w.reshape(K, N), e) <= F32_TOL
+
+
 def test_int8_infinities_nans_and_the_largest_values_read_as_in_f32(dev):
     M, K, N = 40, 300, 200
     rng = np.random.default_rng(3)
@@ -79,7 +101,7 @@ def test_int8_infinities_nans_and_the_largest_values_read_as_in_f32(dev):
 
 
 def test_int8_tiny_activations_keep_f32_accuracy(dev):
-    # the last bf16 term of values near 2^-115 is a bf16 subnormal
+    # unscaled, the last bf16 term of values near 2^-115 would be a bf16 subnormal
     M, K, N = 16, 256, 128
     rng = np.random.default_rng(4)
     a = (rng.standard_normal((M, K)) * 2.0 ** -115).astype(np.float32)
@@ -123,6 +145,20 @@ def test_grouped_f32_matches_the_oracle(dev, form, K, N, counts, T):
             assert rel_l2(got[at:at + c], want) <= F32_TOL, e
         at += c
     assert np.all(got[at:] == (0 if form == "GroupedMatVec" else 7.0))
+
+
+# (exponent of the rows, of the weights)
+@pytest.mark.parametrize("ex,ew", [(e, 0) for e in ENDS] + [(0, e) for e in ENDS] + [(-124, 100), (60, 52)])
+def test_grouped_f32_at_the_ends_of_the_f32_range(dev, ex, ew):
+    E, T, K, N = 2, 40, 256, 96
+    rng = np.random.default_rng(13)
+    x = np.ldexp(rng.standard_normal((T, K)), ex).astype(np.float32)
+    w = np.ldexp(rng.standard_normal((E, K, N)), ew).astype(np.float32)
+    got = grouped_run(dev, "GroupedMatMul", x, w, [20, 20], T, K, N)
+    for e in range(E):
+        rows = slice(20 * e, 20 * e + 20)
+        want = x[rows].astype(np.float64) @ w[e].astype(np.float64)
+        assert scaled_l2(got[rows], want, ex + ew) <= F32_TOL, e
 
 
 @pytest.mark.parametrize("form", ["GroupedMatVec", "GroupedMatMul"])
@@ -262,6 +298,21 @@ def test_int4_rows_of_any_extents_match_the_oracle(dev, M, K, N, bf16):
     want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w + bias
     # bf16: one rounding of the result (2^-9 at most, 2^-9 / sqrt(3) in the norm)
     assert rel_l2(got, want) <= (2.0 ** -9 if bf16 else F32_TOL)
+
+
+@pytest.mark.parametrize("e", ENDS)
+def test_int4_rows_of_any_extents_at_the_ends_of_the_f32_range(dev, e):
+    M, K, N = 20, 300, 203
+    rng = np.random.Generator(np.random.PCG64(14))
+    p, _, _, _ = int4_weights(rng, K, N)
+    groups = -(-K * N // 128)
+    s = oracle.to_f16(np.full(groups, 0.25, np.float32))
+    z = oracle.to_f16(rng.uniform(0, 15, groups).astype(np.float32))
+    w = oracle.int4_dequantize(p, s, z, K * N).astype(np.float64).reshape(K, N)
+    x = np.ldexp(rng.standard_normal((M, K)), e).astype(np.float32)
+    got, launches = int4_run(dev, x, p, s, z, M, K, N)
+    assert launches[0].startswith("split_product_kernel<"), launches
+    assert scaled_l2(got, x.astype(np.float64) @ w, e) <= F32_TOL
 
 
 def test_int4_rows_of_any_extents_infinities(dev):
