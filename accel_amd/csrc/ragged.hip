@@ -19,8 +19,11 @@
 // K is never split across workgroups: no workspace, no hand-off.
 //
 // A weight is (q - z) * s as in the per-element kernels, q - z in f32 and the
-// scale folded into the activation; a zero scale reads as z.  A sum that comes
-// out infinite or NaN is computed again by the per-element loop.
+// scale folded into the activation; a zero scale reads as z.  The fold is with
+// 2^24 s, which is at least 1: an activation times a small scale would go
+// subnormal where its products do not (relative errors of 2e-4 to 2e-3 near
+// 2^-124 with scales of 2^-14).  4096 x 32004 38.7 us without it, 38.9 with.  A
+// sum that comes out infinite or NaN is computed again by the per-element loop.
 //
 // 4096 x 32004 (one row): 1305 us one lane per element, 39 us here (1.7 TB/s).
 #include <hip/hip_runtime.h>
@@ -35,6 +38,7 @@ namespace {
 
 constexpr int kRagThreads = 1024;
 constexpr int kRagBatch = 4;   // rows of a load batch, two batches out at a time
+constexpr float kRagUp = 0x1p24f, kRagDown = 0x1p-24f;   // of the scales folded in
 
 __device__ __forceinline__ float rag_act(float v) { return v; }
 __device__ __forceinline__ float rag_act(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(kRagThreads) void ragged_rows_kernel(
     auto add = [&](const Batch& t) {
 #pragma unroll
         for (int u = 0; u < kRagBatch; u++) {
-            float s = half_bits_to_float(t.s[u]);
+            const float s = half_bits_to_float(t.s[u]) * kRagUp;
             const float z = half_bits_to_float(t.z[u]);
             // a nibble as an e4m3 byte is q 2^-9; the conversion's scale makes
             // it q, exactly
@@ -205,7 +209,8 @@ __global__ __launch_bounds__(kRagThreads) void ragged_rows_kernel(
         if (m >= rows) break;
         if (m) __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 8; j++) red[wave][lane * 8 + j] = acc[m][j] + bias[m];
+        for (int j = 0; j < 8; j++)
+            red[wave][lane * 8 + j] = __builtin_fmaf(acc[m][j], kRagDown, bias[m]);
         __syncthreads();
         // (set of WR waves, lane, j): the waves of the same place in their set
         for (int i = tid; i < WR * 512; i += kRagThreads) {

@@ -277,6 +277,27 @@ def test_int4_rows_whose_scaled_activation_overflows_stay_finite(dev, M):
     assert np.all(np.abs(got - want)[~over] <= bound[~over])
 
 
+@pytest.mark.parametrize("M,bf16", [(1, False), (2, True), (4, False)])
+@pytest.mark.parametrize("e,scale,zero", [(-124, 2.0 ** -14, -500.0), (-115, 2.0 ** -14, -500.0),
+                                          (-126, 0.25, 7.3), (100, 0.25, 7.3), (112, 0.25, 7.3)])
+def test_int4_rows_of_any_width_at_the_ends_of_the_f32_range(dev, M, bf16, e, scale, zero):
+    # an activation times its scale leaves f32's normal numbers before its
+    # products with the weights, scale (code - zero), do
+    K, N = 1000, 203
+    rng = np.random.Generator(np.random.PCG64(15))
+    p, _, _, _ = int4_weights(rng, K, N)
+    groups = -(-K * N // 128)
+    s, z = (oracle.to_f16(np.full(groups, v, np.float32)) for v in (scale, zero))
+    w = oracle.int4_dequantize(p, s, z, K * N).astype(np.float64).reshape(K, N)
+    x = np.ldexp(rng.standard_normal((M, K)), e).astype(np.float32)
+    bits = workloads.bf16_bits(x)
+    got, launches = int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16)
+    assert launches[0].startswith("ragged_rows_kernel<"), launches
+    want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w
+    # bf16: one rounding of a normal result
+    assert scaled_l2(got, want, e) <= (2.0 ** -9 if bf16 else F32_TOL)
+
+
 # (M, K, N): N odd, even and whole groups (there K % 64 != 0 keeps the int4
 # tiles off), K of no whole stage, one row past the few-rows kernel, and the
 # four tiles
