@@ -60,18 +60,21 @@ constexpr float kUp = 0x1p24f, kDown = 0x1p-24f;   // f32 values in the split
 // ---- activations ----------------------------------------------------------
 
 struct ActF32 {
+    static constexpr const char* kName = "ActF32";
     typedef float T;
     static constexpr int kTerms = 3;
     static constexpr float kScale = kUp, kUnscale = kDown;   // of the values split
     static __device__ __forceinline__ float value(T v) { return v; }
 };
 struct ActF16 {
+    static constexpr const char* kName = "ActF16";
     typedef uint16_t T;
     static constexpr int kTerms = 2;
     static constexpr float kScale = 1.0f, kUnscale = 1.0f;
     static __device__ __forceinline__ float value(T v) { return half_bits_to_float(v); }
 };
 struct ActBf16 {
+    static constexpr const char* kName = "ActBf16";
     typedef uint16_t T;
     static constexpr int kTerms = 1;   // itself: not split
     static constexpr float kUnscale = 1.0f;
@@ -99,6 +102,7 @@ struct F32W {
     using One = F32W<kOne>;
     One one() const { return {w}; }
     static constexpr float kUnscale = kDown;
+    static std::string name() { return tname("F32W", FORM); }   // as a kernel trace shows it
     const float* w;
     __device__ __forceinline__ F32W expert(int e, size_t per) const { return {w + e * per}; }
     struct Regs { float v[8][2]; };
@@ -120,9 +124,6 @@ struct F32W {
         if constexpr (FORM != kOne) w1 = r.v[i][1] * kUp;
     }
     __device__ __forceinline__ float at(uint64_t f) const { return w[f]; }
-    static std::string grouped_name(int tm, int wn, int kg) {
-        return tname("split_grouped_kernel", "F32W", tm, wn, kg);
-    }
 };
 
 template <int FORM>
@@ -130,6 +131,7 @@ struct Int8W {
     using One = Int8W<kOne>;
     One one() const { return {q, s}; }
     static constexpr float kUnscale = 1.0f;   // a weight is 0 or at least 2^-24
+    static std::string name() { return tname("Int8W", FORM); }
     const int8_t* q;
     const uint16_t* s;
     struct Regs { uint32_t q[8], s[8], q1[8], s1[8]; };   // q1, s1: odd N only
@@ -175,6 +177,7 @@ struct Int4W {
     using One = Int4W<kOne>;
     One one() const { return {c, s, z}; }
     static constexpr float kUnscale = 1.0f;   // a weight is 0 or at least 2^-48
+    static std::string name() { return tname("Int4W", FORM); }
     const uint8_t* c;      // two codes a byte, low nibble first
     const uint16_t* s;
     const uint16_t* z;
@@ -229,9 +232,6 @@ struct Int4W {
         const float sv = half_bits_to_float(s[f >> 7]), zv = half_bits_to_float(z[f >> 7]);
         const uint32_t code = (c[f >> 1] >> (4 * (f & 1))) & 15u;
         return sv == 0.0f ? zv : ((float)code - zv) * sv;
-    }
-    static std::string grouped_name(int tm, int wn, int kg) {
-        return tname("split_grouped_kernel", "Int4W", tm, wn, kg);
     }
 };
 
@@ -686,7 +686,8 @@ hipError_t launch_split_tile(hipStream_t st, const typename ACT::T* a, W w, void
     using S = Shape<ACT, TM, WN, KG>;
     const long long tiles =
         (long long)((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN);
-    ACCEL_LAUNCH(tname("split_product_kernel", TM, WN, KG) + grid_note(tiles, 1),
+    ACCEL_LAUNCH(tname("split_product_kernel", W::name().c_str(), ACT::kName, TM, WN, KG) +
+                     grid_note(tiles, 1),
                  (split_product_kernel<W, ACT, TM, WN, KG>),
                  dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(S::NT), 0, st, a, w, out, M, K, N, ep);
     return launch_status();
@@ -724,7 +725,8 @@ hipError_t launch_grouped_tile(hipStream_t st, const typename ACT::T* x, W w, co
                                float* out, int E, int T, int K, int N, bool matvec) {
     using S = Shape<ACT, TM, WN, KG>;
     const long long wgs = most_blocks(T, E, S::BM) * ((N + S::BN - 1) / S::BN);
-    ACCEL_LAUNCH(W::grouped_name(TM, WN, KG), (split_grouped_kernel<W, ACT, TM, WN, KG>),
+    ACCEL_LAUNCH(tname("split_grouped_kernel", W::name().c_str(), ACT::kName, TM, WN, KG),
+                 (split_grouped_kernel<W, ACT, TM, WN, KG>),
                  dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(S::NT), 0, st, x, w, off, out, E, T, K,
                  N, matvec);
     return launch_status();

@@ -215,19 +215,22 @@ def test_prepared_rows_need_even_k_and_aligned_rows():
     (1, 4096, 32004, A.F32, "ragged_rows_kernel<float, 1, 32>"),
     (1, 128, 64, A.BF16, "ragged_rows_kernel<unsigned short, 1, 8>"),
     (3, 1000, 15001, A.F32, "ragged_rows_kernel<float, 4, 16>"),
-    (5, 1000, 1001, A.F32, "split_product_kernel<1, 1, 16>"),
-    (100, 4100, 4004, A.F32, "split_product_kernel<1, 1, 8>"),
-    (512, 4100, 4096, A.BF16, "split_product_kernel<2, 2, 4>"),
+    (5, 1000, 1001, A.F32, "split_product_kernel<Int4W<3>, ActF32, 1, 1, 16>"),
+    (100, 4100, 4004, A.F32, "split_product_kernel<Int4W<1>, ActF32, 1, 1, 8>"),
+    (512, 4100, 4096, A.BF16, "split_product_kernel<Int4W<2>, ActBf16, 2, 2, 4>"),
     (17, 127, 128, A.F32, "int4_gemm_f32_kernel"),
     (1, 128, 63, A.F32, "int4_generic_f32_kernel"),
     (1, 31, 100, A.F32, "int4_generic_f32_kernel"),
-    (9, 32, 66, A.BF16, "split_product_kernel<1, 1, 8>"),
+    (9, 32, 66, A.BF16, "split_product_kernel<Int4W<1>, ActBf16, 1, 1, 8>"),
+    (9, 32, 66, A.F32, "split_product_kernel<Int4W<1>, ActF32, 1, 1, 8>"),
+    (100, 4100, 4003, A.F32, "split_product_kernel<Int4W<0>, ActF32, 1, 1, 8>"),
 ])
 def test_matrices_of_any_extents(M, K, N, dtype, name):
     """Widths that are no multiple of a group and depths no tile takes: up to
     four rows on the column strips, more on the tiles of split weights; below
     64 columns or 32 rows (128 where N is whole groups), or off 16-byte
-    alignment, as before."""
+    alignment, as before.  The tiles' names carry their weights' form and the
+    rows' type, as a kernel trace does."""
     sel = A.select(M, K, N, dtype, a=ALIGNED, codes=ALIGNED)
     assert _names(sel) == [name], sel
     off = A.select(M, K, N, dtype, a=ALIGNED + 4, codes=ALIGNED)
