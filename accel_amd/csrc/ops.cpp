@@ -979,10 +979,17 @@ int run_grouped_int4(const char* op, int dev, void* stream, const accel_tensor_t
                  "each expert's 128-row blocks";
         rejected = "the decode kernels: they take at most 1024 f32 rows";
     } else if (f32) {
-        reason = "f32 rows no int4 tile takes: the matrix-core tiles of split weights (rows and "
-                 "dequantised weights in three bf16 terms each), any extents and offsets";
         rejected = "the f32 matrix-core tiles: they take K % 64 == 0, N % 128 == 0 and "
-                   "16-byte aligned rows; the decode kernels: at most 1024 rows";
+                   "16-byte aligned rows; the decode kernels: they take at most 1024 rows, N a "
+                   "multiple of 128 and 16-byte aligned codes";
+        if (split_grouped_supported((int)experts, (int)T, (int)K, (int)N)) {
+            reason = "f32 rows no int4 tile takes: the matrix-core tiles of split weights (rows "
+                     "and dequantised weights in three bf16 terms each), any offsets";
+        } else {
+            reason = "extents no tile takes: one lane per (row, column)";
+            rejected += "; the tiles of split weights: they take N <= 2^24, K < 2^30 and at most "
+                        "2^21 tiles of 32 x 32";
+        }
     } else {
         reason = "bf16 rows: the matrix-core tiles walking each expert's blocks of up to 256 "
                  "rows";

@@ -374,6 +374,31 @@ def test_int4_grouped_of_any_width_matches_the_oracle(dev, form, K, N, counts, T
             assert np.all(got[t] == (0 if form == "Int4GroupedMatVec" else 7.0)), t
 
 
+# Past the tiles' widths (N <= 2^24) the kernels of one lane, or one small f32
+# tile, per element still run.
+
+def test_int4_grouped_past_the_tiles_widths_says_so_and_matches_the_oracle(dev):
+    E, T, K, N = 2, 3, 2, (1 << 24) + 64
+    rng = np.random.Generator(np.random.PCG64(16))
+    groups = E * K * N // 128
+    p = rng.integers(0, 1 << 32, E * K * N // 8, dtype=np.uint64).astype(np.uint32)
+    s = oracle.to_f16(rng.uniform(0.01, 0.02, groups).astype(np.float32))
+    z = oracle.to_f16(rng.uniform(0, 15, groups).astype(np.float32))
+    w = oracle.int4_dequantize(p, s, z, E * K * N).reshape(E, K, N)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    xb, wd = dev.upload(x), dev.upload_int4(p, s, z, E * K * N)
+    cb, ob = dev.upload(np.array([2, 1], np.uint32), U32), dev.alloc((T, N), F32)
+    dev.Int4GroupedMatMul(xb, wd, E, cb, ob)
+    got, sel = ob.numpy(), dev.last_selection()
+    for b in (xb, wd, cb, ob):
+        b.free()
+    assert sel.launches[-1].startswith("grouped_f32_kernel<true>"), sel
+    assert "one lane per" in sel.reason and "split" not in sel.reason, sel
+    assert any("tiles of split weights" in r for r in sel.rejected), sel
+    for t, e in enumerate((0, 0, 1)):
+        assert rel_l2(got[t], x[t].astype(np.float64) @ w[e]) <= F32_TOL, t
+
+
 @pytest.mark.parametrize("n", [2047, 2048, 2049, 16384 + 1920, 3 * 2048 + 128 * 5 + 77])
 def test_packer_waves_of_sixteen_groups_are_bit_exact(dev, n):
     """Whole waves beside single groups, and waves that leave the fast path:
