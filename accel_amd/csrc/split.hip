@@ -252,7 +252,7 @@ struct Shape {
     static constexpr int BUF = NA * 4 * OCT;
     // a one-wave group reads its own chunks only: no second buffer needed
     static constexpr int BUFS = WN == 1 ? 1 : 2;
-    static constexpr int SUM_BYTES = KG > 1 ? KG * BM * BN * 4 : 0;
+    static constexpr int SUM_BYTES = KG * BM * BN * 4;
     static constexpr int LDS = KG * BUFS * BUF > SUM_BYTES ? KG * BUFS * BUF : SUM_BYTES;
 };
 
@@ -506,50 +506,34 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
         }
     }
 
-    // out, through LDS in K group order when there are several
+    // out, through LDS in K group order
     constexpr float kBack = ACT::kUnscale * W::kUnscale;
     float odd = 0.0f;   // becomes NaN when a sum is not finite
     const int rows = min(BM, m_end - m0), cols = min(BN, N - n0);
-    if constexpr (KG == 1) {
+    __syncthreads();   // every group has left its last stage
+    float* sums = reinterpret_cast<float*>(lds);
 #pragma unroll
-        for (int t = 0; t < TM; t++)
+    for (int t = 0; t < TM; t++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int rl = t * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-                    if (rl < rows && cp + j < cols) {
-                        const float v = acc[t][j][r] * kBack;
-                        odd = __builtin_fmaf(v, 0.0f, odd);
-                        store_out(out, (size_t)(m0 + rl) * N + n0 + cp + j, n0 + cp + j, v, ep);
-                    }
-            }
-    } else {
-        __syncthreads();   // every group has left its last stage
-        float* sums = reinterpret_cast<float*>(lds);
-#pragma unroll
-        for (int t = 0; t < TM; t++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int rl = t * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
-                float* at = sums + (g * BM + rl) * BN + cp;
-                if constexpr (TN == 2)
-                    *reinterpret_cast<f32x2*>(at) = (f32x2){acc[t][0][r], acc[t][TN - 1][r]};
-                else
-                    *at = acc[t][0][r];
-            }
-        __syncthreads();
+        for (int r = 0; r < 16; r++) {
+            const int rl = t * 32 + 8 * (r >> 2) + 4 * kg + (r & 3);
+            float* at = sums + (g * BM + rl) * BN + cp;
+            if constexpr (TN == 2)
+                *reinterpret_cast<f32x2*>(at) = (f32x2){acc[t][0][r], acc[t][TN - 1][r]};
+            else
+                *at = acc[t][0][r];
+        }
+    __syncthreads();
 #pragma unroll 4
-        for (int i = tid; i < BM * BN; i += S::NT) {
-            const int rl = i / BN, cl = i % BN;
-            float v = sums[i];
+    for (int i = tid; i < BM * BN; i += S::NT) {
+        const int rl = i / BN, cl = i % BN;
+        float v = sums[i];
 #pragma unroll
-            for (int q = 1; q < KG; q++) v += sums[q * BM * BN + i];
-            v *= kBack;
-            if (rl < rows && cl < cols) {
-                odd = __builtin_fmaf(v, 0.0f, odd);
-                store_out(out, (size_t)(m0 + rl) * N + n0 + cl, n0 + cl, v, ep);
-            }
+        for (int q = 1; q < KG; q++) v += sums[q * BM * BN + i];
+        v *= kBack;
+        if (rl < rows && cl < cols) {
+            odd = __builtin_fmaf(v, 0.0f, odd);
+            store_out(out, (size_t)(m0 + rl) * N + n0 + cl, n0 + cl, v, ep);
         }
     }
     if (__syncthreads_or(odd != 0.0f)) {
