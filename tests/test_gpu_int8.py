@@ -7,7 +7,8 @@ and QuantMatMulTiledF32 (internal/kernels/quant.go:195-238); inputs whose
 every product and partial sum is exact in f32 (the reference's
 prefill_test.go:934-960 style) are compared exactly.  Both kernels run: the
 decode kernel (M <= 8, N a multiple of 256, 16-byte aligned quants) and the
-tiled kernel (everything else).
+matrix-core tiles of split weights (everything else; each of those tiles, and
+the kernel past their widths, in test_gpu_split.py).
 """
 import ctypes
 import struct

@@ -14,7 +14,8 @@ inputs, and within one bf16 rounding of it elementwise.
 Shapes cover every kernel the product routes to: the VALU decode kernel
 (M = 1, 2, and 9..16 rows as eight plus the rest), the matrix-core decode
 kernel (M = 3..16), the f32 tiled kernel (M > 16), the per-element kernels
-(ragged N) and the bf16 matrix-core tiles.
+(N below 64) and the bf16 matrix-core tiles.  The kernels of other widths are in
+test_gpu_split.py.
 """
 import numpy as np
 import pytest

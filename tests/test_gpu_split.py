@@ -1,10 +1,13 @@
 """GPU parity of the matrix-core products of split weights (split.hip): every
-tile, the ragged ends of rows, columns and K, every K-group remainder, and
-infinities, NaNs and tiny values.
+tile (asserted by name), the ragged ends of rows, columns and K, every K-group
+remainder, and infinities, NaNs and tiny values; and of the column strips
+(ragged.hip).
 
 Tolerance: rel-L2 1e-5 against the oracle, the path's bound for f32 products.
 The split itself is within 2^-26 of each product; both sides round their sums.
 """
+import re
+
 import numpy as np
 import pytest
 
@@ -16,6 +19,8 @@ from conftest import rel_l2
 pytestmark = pytest.mark.gpu
 
 F32_TOL = 1e-5
+# one rounding to bf16 of an f32 result: half a unit of 8 bits is 2^-8 of a value at most
+BF16_ROUND = 2.0 ** -8 + F32_TOL
 
 
 def int8_run(dev, a, q, s, M, K, N, f16=False):
@@ -30,7 +35,7 @@ def int8_run(dev, a, q, s, M, K, N, f16=False):
 
 # (M, K, N): K of no whole stage, fewer stages than K groups, a ragged last
 # stage; one row, one column, column pairs cut by the edge; N odd, even and
-# whole blocks; the tiles 32 x 64, 64 x 64, 64 x 128 and 64 x 256
+# whole blocks (which tile: TILES below)
 INT8 = [(9, 1, 1), (9, 31, 33), (33, 32, 64), (10, 95, 130), (64, 257, 65), (31, 300, 2),
         (2, 1656, 1359), (130, 511, 96), (257, 1000, 1500), (100, 4100, 4004),
         (512, 1024, 8192), (2048, 260, 8190), (65, 4097, 16383)]
@@ -48,6 +53,36 @@ def test_int8_matches_the_oracle(dev, M, K, N, f16):
     x = (oracle.f16_to_f32(a) if f16 else a).astype(np.float64).reshape(M, K)
     w = q.astype(np.float64) * oracle.f16_to_f32(s).astype(np.float64)[np.arange(K * N) // 32]
     assert rel_l2(got, x @ w.reshape(K, N)) <= F32_TOL
+
+
+# The five tiles, (32-row m-tiles, waves across the columns, K groups), and rows,
+# depth and width that the cost rule gives each on the MI355X's 256 CUs, also a
+# few columns either way.
+TILES = [((2, 1, 8), 250, 300, 4000), ((2, 2, 4), 400, 300, 4000), ((2, 4, 2), 500, 160, 8000),
+         ((1, 1, 8), 100, 300, 4000), ((1, 1, 16), 33, 300, 1000)]
+TILE_IDS = ["64x64", "64x128", "64x256", "32x64", "32x32"]
+
+
+def tile_of(sel):
+    """The tile of a split product's launch, from its reported name."""
+    found = [re.match(r"split_(?:product|grouped)_kernel<.*, (\d+), (\d+), (\d+)>", k)
+             for k in sel.launches]
+    return next((tuple(int(v) for v in m.groups()) for m in found if m), None)
+
+
+def planned_tile(M, K, N):
+    """The tile of an M x K x N product of split weights: the rule looks at the
+    extents alone, so an int4 product of an even width next to N's reports it."""
+    return tile_of(accel_amd.select(M, K, N + N % 2, F32))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("more", [0, 1, 2])   # whole blocks of 32, odd, even
+@pytest.mark.parametrize("tile,M,K,N", TILES, ids=TILE_IDS)
+def test_int8_on_every_tile_matches_the_oracle(dev, tile, M, K, N, more, f16):
+    N += more - (8 if N == 1000 else 0)       # 992 is whole blocks
+    assert planned_tile(M, K, N) == tile
+    test_int8_matches_the_oracle(dev, M, K, N, f16)
 
 
 # Activations near the ends of the f32 range, weights of ordinary size: the
@@ -124,7 +159,7 @@ def grouped_run(dev, form, x, w, counts, T, K, N):
 
 
 # (K, N, counts, T): one row, empty experts, blocks that end in one row, rows
-# past the last segment, N odd and even, K of no whole stage, the four tiles
+# past the last segment, N odd and even, K of no whole stage
 GROUPED = [(7, 1, [1], 1), (100, 33, [0, 5, 0, 65], 73), (64, 130, [1, 0, 0, 1], 3),
            (257, 64, [64, 1, 33, 0], 98), (300, 1022, [129, 3], 140), (1024, 2048, [70, 90, 60], 220),
            (32, 24000, [200, 300, 140, 1], 641), (130, 1000, [0, 0, 0], 5)]
@@ -145,6 +180,40 @@ def test_grouped_f32_matches_the_oracle(dev, form, K, N, counts, T):
             assert rel_l2(got[at:at + c], want) <= F32_TOL, e
         at += c
     assert np.all(got[at:] == (0 if form == "GroupedMatVec" else 7.0))
+
+
+# The same for the grouped products: half of the tokens in one expert, the depth
+# whole groups whatever the width.
+GROUPED_TILES = [((2, 1, 8), 2, 128, 256, 4000), ((2, 2, 4), 8, 256, 256, 4000),
+                 ((2, 4, 2), 4, 640, 128, 4000), ((1, 1, 8), 2, 90, 256, 4000),
+                 ((1, 1, 16), 2, 6, 512, 1000)]
+
+
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("tile,E,T,K,N", GROUPED_TILES, ids=TILE_IDS)
+def test_grouped_products_on_every_tile_match_the_oracle(dev, tile, E, T, K, N, odd):
+    rng = np.random.Generator(np.random.PCG64(T + odd))
+    counts = [T // 2] + [(T - T // 2) // (E - 1)] * (E - 1)
+    counts[-1] += T - sum(counts)
+    # int4 experts of an even width, whose report names the tile
+    p, s, z, w = int4_weights(rng, E * K, N + 2 * odd)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    xb, wd = dev.upload(x), dev.upload_int4(p, s, z, w.size)
+    cb, ob = dev.upload(np.array(counts, np.uint32), U32), dev.alloc((T, N + 2 * odd), F32)
+    dev.Int4GroupedMatMul(xb, wd, E, cb, ob)
+    got4, sel = ob.numpy(), dev.last_selection()
+    for b in (xb, wd, cb, ob):
+        b.free()
+    assert tile_of(sel) == tile, sel
+    # f32 experts: the same rule, the same extents (odd: one column less)
+    wf = (rng.standard_normal((E, K, N + odd)) * 0.05).astype(np.float32)
+    got = grouped_run(dev, "GroupedMatMul", x, wf, counts, T, K, N + odd)
+    w, at = w.reshape(E, K, N + 2 * odd), 0
+    for e, c in enumerate(counts):
+        xe = x[at:at + c].astype(np.float64)
+        assert rel_l2(got4[at:at + c], xe @ w[e]) <= F32_TOL, e
+        assert rel_l2(got[at:at + c], xe @ wf[e].astype(np.float64)) <= F32_TOL, e
+        at += c
 
 
 # (exponent of the rows, of the weights)
@@ -244,6 +313,24 @@ def test_int4_matvec_of_any_width_matches_the_oracle(dev, K, N):
         assert rel_l2(got, want if M > 1 or bf16 else want[0]) <= (4e-3 if bf16 else F32_TOL), (M, bf16)
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 33, 65), (2, 130, 203), (4, 511, 1001), (3, 130, 14401)])
+def test_int4_linear_of_few_rows_of_any_width_adds_the_bias(dev, M, K, N, bf16):
+    rng = np.random.Generator(np.random.PCG64(M * 31 + N))
+    p, s, z, w = int4_weights(rng, K, N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias = (100 * rng.standard_normal(N)).astype(np.float32)
+    bits = workloads.bf16_bits(x)
+    run = lambda b: int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16, "Int4Linear", b)  # noqa: E731
+    got, launches = run(bias)
+    assert launches[0].startswith("ragged_rows_kernel<"), launches
+    if not bf16:
+        # one f32 addition to what the product alone stores
+        assert np.array_equal(got, run(None)[0] + bias)
+    want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w + bias
+    assert rel_l2(got, want) <= (BF16_ROUND if bf16 else F32_TOL)
+
+
 def test_int4_matvec_of_any_width_infinities_and_nans(dev):
     K, N = 300, 203
     rng = np.random.Generator(np.random.PCG64(9))
@@ -294,13 +381,11 @@ def test_int4_rows_of_any_width_at_the_ends_of_the_f32_range(dev, M, bf16, e, sc
     got, launches = int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16)
     assert launches[0].startswith("ragged_rows_kernel<"), launches
     want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w
-    # bf16: one rounding of a normal result
-    assert scaled_l2(got, want, e) <= (2.0 ** -9 if bf16 else F32_TOL)
+    assert scaled_l2(got, want, e) <= (BF16_ROUND if bf16 else F32_TOL)
 
 
 # (M, K, N): N odd, even and whole groups (there K % 64 != 0 keeps the int4
-# tiles off), K of no whole stage, one row past the few-rows kernel, and the
-# four tiles
+# tiles off), K of no whole stage, and one row past the few-rows kernel
 INT4 = [(5, 128, 65), (6, 129, 64), (9, 32, 66), (40, 47, 333), (33, 200, 1001), (17, 511, 130), (64, 1000, 999),
         (100, 4100, 4004), (40, 136, 384), (70, 2090, 256), (513, 260, 8190), (300, 1026, 4098),
         (65, 130, 16391)]
@@ -317,8 +402,21 @@ def test_int4_rows_of_any_extents_match_the_oracle(dev, M, K, N, bf16):
     got, launches = int4_run(dev, bits if bf16 else x, p, s, z, M, K, N, bf16, "Int4Linear", bias)
     assert launches[0].startswith("split_product_kernel<"), launches
     want = (workloads.bf16_to_f32(bits) if bf16 else x).astype(np.float64) @ w + bias
-    # bf16: one rounding of the result (2^-9 at most, 2^-9 / sqrt(3) in the norm)
+    # bf16: one rounding of the result (2^-8 at most, 2^-9.2 in the norm of many values)
     assert rel_l2(got, want) <= (2.0 ** -9 if bf16 else F32_TOL)
+
+
+# Even widths and whole groups (where the 64-column tiles start halfway through
+# one) on every tile; odd widths take the 32-row tiles alone.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("form", ["odd", "even", "groups"])
+@pytest.mark.parametrize("tile,M,K,N", TILES, ids=TILE_IDS)
+def test_int4_on_every_tile_matches_the_oracle(dev, tile, M, K, N, form, bf16):
+    N = {"odd": N + 1, "even": N + 2, "groups": (N + 64) // 128 * 128}[form]
+    sel = accel_amd.select(M, K, N, BF16 if bf16 else F32)
+    want = tile if form != "odd" or tile == (1, 1, 16) else (1, 1, 8)
+    assert tile_of(sel) == want, sel
+    test_int4_rows_of_any_extents_match_the_oracle(dev, M, K, N, bf16)
 
 
 @pytest.mark.parametrize("e", ENDS)
@@ -397,6 +495,16 @@ def test_int4_grouped_past_the_tiles_widths_says_so_and_matches_the_oracle(dev):
     assert any("tiles of split weights" in r for r in sel.rejected), sel
     for t, e in enumerate((0, 0, 1)):
         assert rel_l2(got[t], x[t].astype(np.float64) @ w[e]) <= F32_TOL, t
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_int8_past_the_tiles_widths_matches_the_oracle(dev, f16):
+    test_int8_matches_the_oracle(dev, 2, 3, (1 << 24) + 1, f16)
+
+
+def test_grouped_f32_past_the_tiles_widths_matches_the_oracle(dev):
+    for form in ("GroupedMatVec", "GroupedMatMul"):
+        test_grouped_f32_matches_the_oracle(dev, form, 2, (1 << 24) + 1, [2, 1], 4)
 
 
 @pytest.mark.parametrize("n", [2047, 2048, 2049, 16384 + 1920, 3 * 2048 + 128 * 5 + 77])

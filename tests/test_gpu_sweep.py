@@ -5,7 +5,8 @@ sweeps draw (rows, K, N, dtype, form) at random from pools that cross every
 route boundary the launchers have: one and two rows (VALU decode), 3..16 rows
 (matrix-core decode), 17+ rows (prefill tiles, split K when the tiles are
 few), K and N that are and are not multiples of the tiles' 64 and 128 (the
-generic kernels, groups that span rows), and 256 / 512-column decode tiles.
+column strips, the tiles of split weights and the per-element kernels; groups
+that span rows), and 256 / 512-column decode tiles.
 Every case is checked against the oracle at the path's tolerance (rel-L2 1e-5
 for f32, 2e-2 for bf16, as `tensor/int4_test.go:275-354` and
 `tensor/grouped_test.go:20-283` check their products).  Each case prints its
@@ -90,8 +91,8 @@ GROUPED_N = [128, 256, 384, 512, 1024, 8192]
 def test_random_grouped_shapes_match_the_oracle(dev, seed):
     """Ragged expert counts (empty experts, padding rows past the last
     segment), both forms, both activation dtypes of the int4 grouped products:
-    the decode-MoE kernel (f32, up to 64 rows), the lane-per-element form (f32,
-    more rows) and the matrix-core grouped tiles (bf16)."""
+    the decode-MoE kernels (up to 1024 f32 or 64 bf16 rows) and the matrix-core
+    grouped tiles (more)."""
     rng = np.random.Generator(np.random.PCG64(2000 + seed))
     done = 0
     while done < 10:
