@@ -13,9 +13,10 @@
 // their last bit, 2^-149, among bf16's normal numbers, and the sums are scaled
 // back (exact but for results that are subnormal).  Without it relative errors
 // were 4e-5 at 2^-120 and 2e-3 at 2^-126.  It costs a multiplication an f32
-// value (us without / with, one card): int8 512 x 4096 x 4096 97.9 / 98.7, 256
-// rows of 8 f32 experts of 2048 x 4096 73.9 / 74.6, int4 100 x 4100 x 4004
-// 48.0 / 49.1.  Operands from 2^104 on (sums from 2^80 with f32 experts) leave
+// value, 1-2% and up to 6% where the narrow tile splits few rows (us without /
+// with, one card): int8 512 x 4096 x 4096 92.7 / 94.0, 256 rows of 8 f32 experts
+// of 2048 x 4096 71.9 / 73.0, int4 100 x 4100 x 4004 46.3 / 46.8, int8 33 x 4864
+// x 352 29.9 / 31.5, 8 rows of 4 f32 experts of 156 x 2397 10.7 / 11.3.  Operands from 2^104 on (sums from 2^80 with f32 experts) leave
 // the range and are computed again as below.
 //
 // Bound: the matrix cores, at three to six times the product's flops; for few
@@ -120,8 +121,12 @@ struct F32W {
         }
     }
     __device__ __forceinline__ void pair(Regs& r, int i, int, float& w0, float& w1) const {
+        asm volatile("" : "+v"(r.v[i][0]));   // as in Int8W
         w0 = r.v[i][0] * kUp;
-        if constexpr (FORM != kOne) w1 = r.v[i][1] * kUp;
+        if constexpr (FORM != kOne) {
+            asm volatile("" : "+v"(r.v[i][1]));
+            w1 = r.v[i][1] * kUp;
+        }
     }
     __device__ __forceinline__ float at(uint64_t f) const { return w[f]; }
 };
@@ -332,9 +337,13 @@ __device__ __forceinline__ void split_tile(char* lds, const typename ACT::T* __r
     auto split_a = [&](int u, int p) {   // pair p of unit u
         if constexpr (NA == 1)
             ta[p][0] = (uint32_t)ra[u][2 * p] | ((uint32_t)ra[u][2 * p + 1] << 16);
-        else
+        else {
+            // marked like the weights (Int8W::pair): scaled where they are split
+            if constexpr (ACT::kScale != 1.0f)
+                asm volatile("" : "+v"(ra[u][2 * p]), "+v"(ra[u][2 * p + 1]));
             split_terms<NA>(ACT::value(ra[u][2 * p]) * ACT::kScale,
                             ACT::value(ra[u][2 * p + 1]) * ACT::kScale, ta[p]);
+        }
     };
     auto write_a = [&](int u, int buf) {
         const int row = a_row + u * (TG / 4);
