@@ -145,7 +145,7 @@ hipError_t launch_grouped_f32(const Device* d, hipStream_t st, const float* x, c
                               bool write_padding) {
     if (T == 0 || N == 0) return hipSuccess;
     // The matrix-core tiles wherever their grid reaches (us, one lane per
-    // element / tiles): 256 rows of 8 experts of 2048 x 4096 1536 / 65, 8 rows
+    // element / tiles): 256 rows of 8 experts of 2048 x 4096 1533 / 68, 8 rows
     // of 4 experts of 156 x 2397 42 / 11.
     if (split_grouped_supported(E, T, K, N))
         return launch_split_grouped_f32(d, st, x, w, off, out, E, T, K, N, write_padding);

@@ -286,8 +286,8 @@ hipError_t launch_int8_any(Device* d, hipStream_t st, const ACT* a, const int8_t
             default: return launch_int8_decode_m<8>(d, st, a, q, s, out, K, N, status);
         }
     }
-    // The matrix-core tiles past the decode shapes: 512 x 4096 x 4096 702 -> 90
-    // us, up to 32 rows 27, 155 x 1758 x 430 (f32 VALU tiles / here) 98 / 20; the
+    // The matrix-core tiles past the decode shapes: 512 x 4096 x 4096 704 -> 93
+    // us, up to 32 rows 27, 155 x 1758 x 430 (f32 VALU tiles / here) 98 / 18; the
     // decode kernel keeps its eight rows (15.6 us there, 27 here).
     if (split_product_supported(M, K, N))
         return launch_split_int8(d, st, a, sizeof(ACT) == 2, q, s, out, M, K, N);

@@ -389,9 +389,9 @@ hipError_t launch_split_grouped_f32(const Device* d, hipStream_t st, const float
 // fp32 VALU tiles hold) at 16-byte aligned addresses (us, one lane per element
 // or VALU tiles / here): 1 x 32 x 1001 6.4 / 5.6, 2 x 64 x 65 8.5 / 5.5, 192 x
 // 111 x 555 20 / 9.8, 40 x 130 x 256 19.5 / 8.9, but 300 x 16 x 1000 5.5 / 5.9.
-// Below that a launch is mostly empty;
-// rows or codes from other addresses keep the kernels that load single
-// elements.
+// Below that a launch is mostly empty.  Rows or codes from other addresses keep
+// the kernels of one lane per element; the tiles and strips load single elements
+// too and have not been timed there.
 bool int4_ragged_shape(const void* a, const void* codes, int K, int N);
 // Up to four rows of f32 or bf16 (out then bf16) on a matrix whose width is
 // no multiple of a group: ragged.hip, no workspace.

@@ -1,9 +1,12 @@
 // Int4MatVec and Int4MatMul of up to four rows on matrices whose width is no
 // multiple of a quantisation group, so groups and code words run across rows.
 //
-// Bound: instruction issue (about 60 a lane's word, 3 cycles each) and, with
-// narrow strips over the whole chip, L2: a row's scale and zero are a 128-byte
-// line each for two bytes.
+// Bound: one workgroup's instruction issue (about 60 a lane's word, 3 cycles
+// each).  A strip walks all of K, so its time hardly depends on how many there
+// are: 248 columns of 4096 rows take 38.5 us with 17 of them and 38.9 with 154,
+// and the CUs past the strips' number are idle (126 of 256 at 32004 columns).
+// Narrow strips over the whole chip meet L2 as well: a row's scale and zero are a
+// 128-byte line each for two bytes.
 //
 // Row k's columns begin at nibble k N, so what a code word means for a column
 // depends on k N mod 8 only.  A workgroup of 1024 lanes owns a strip of columns
@@ -250,8 +253,8 @@ void launch_ragged(hipStream_t st, const XT* a, Int4Planes w, void* out, int row
 // The strip: narrow strips end sooner (fewer row steps a lane), wide ones share
 // their rows' scale and zero lines among more columns; the narrowest whose
 // strips are one round of the chip, else the widest.  One row, 56 / 120 / 248
-// columns (us): 4096 x 4004 15 / 21 / 38, 4096 x 16001 34 / 23 / 38, 4096 x
-// 32004 63 / 52 / 44.
+// columns (us): 4096 x 4004 15.6 / 21.3 / 38.5, 4096 x 16001 33.3 / 23.4 / 39.0,
+// 4096 x 30001 49.0 / 25.0 / 38.8, 4096 x 32004 46.2 / 41.2 / 38.9.
 template <typename XT, int M>
 void launch_ragged_strip(const Device* d, hipStream_t st, const XT* a, Int4Planes w, void* out,
                          int rows, int K, int N, Epilogue ep) {

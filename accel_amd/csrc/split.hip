@@ -639,12 +639,24 @@ __global__ __launch_bounds__((Shape<ACT, TM, WN, KG>::NT), (KG == 16 ? 4 : 2)) v
 }
 
 // Which tile: the tiles in rounds of the chip, times a K group's stages, times
-// what a stage costs.  The stage costs are measured (us, K = 4096, every CU
-// busy): a wide tile splits its activations for more columns, a narrow one
-// fills the chip with fewer rows and columns.  int8, K = N = 4096 (us), tiles
-// of 64 x 256, 64 x 128, 64 x 64, 32 x 64 and 32 x 32: 512 rows 151, 96, 131,
-// 163, 229; 128 rows 134, 73, 46, 37, 54; 32 rows 132, 73, 46, 35, 27; and 33 x
-// 4864 x 352 157, 86, 52, 40, 30.
+// what a stage costs.  The stage costs are those of int8 weights and f32 rows
+// (us, K = 4096, every CU busy): a wide tile splits its activations for more
+// columns, a narrow one fills the chip with fewer rows and columns.  The other
+// sources cost more or less a stage but keep the order.  Tiles of 64 x 256, 64 x
+// 128, 64 x 64, 32 x 64 and 32 x 32 (us), the chosen one marked:
+//   int8, f32 rows, K = N = 4096: 512 rows 137, 96*, 116, 154, 229; 128 rows 135,
+//     77, 48, 38*, 56; 32 rows 134, 76, 47, 35, 27*; 33 x 4864 x 352 157, 88, 54,
+//     40, 32*
+//   int8, f16 rows, K = N = 4096: 512 rows 118, 79*, 93, 127, 191
+//   int4, f32 rows, 4100 x 4004: 512 rows 170, 111*, 134, 186, 290; 256 rows 169,
+//     98, 68*, 93, 142; 100 rows 169, 98, 60, 47*, 69; 32 rows 167, 97, 59, 46, 35*
+//   int4, bf16 rows, 4100 x 4004: 512 rows 135, 75*, 89, 155, 225; 100 rows 134,
+//     72, 43, 40*, 56; 32 rows 132, 70, 42, 40, 29*
+//   8 f32 experts of 2048 x 4096: 256 rows 78, 73*, 82, 89, 115; 1024 rows 166,
+//     159*, 184, 215, 308
+// Few rows of many experts are where it misses, its row blocks being an estimate
+// there: 60 rows of the same experts 76, 70, 79, 67, 79*; 16 rows of 4 of 1000 x
+// 3000 43, 30, 24, 20, 25*.
 enum class SplitTile { k64x256, k64x128, k64x64, k32x64, k32x32 };
 
 SplitTile choose_tile(const Device* d, long long rows_blocks64, long long rows_blocks32, int K,
